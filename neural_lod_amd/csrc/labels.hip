@@ -55,6 +55,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "kernels.h"
@@ -124,15 +125,25 @@ __device__ v3 sphere_dir(uint64_t& st) {
     return {a / r, b / r, c / r};
 }
 
-// Moller-Trumbore: t of the hit, or a negative value / NaN for none.
-__device__ __forceinline__ float ray_triangle(v3 o, v3 d, const float* tri) {
+// A triangle as its first vertex and two edges.
+struct Tri {
+    v3 p0, e1, e2;
+};
+
+__device__ __forceinline__ Tri load_tri(const float* __restrict__ tris, uint32_t t) {
+    const float* tri = tris + (size_t)t * 9;
     const v3 p0 = {tri[0], tri[1], tri[2]}, p1 = {tri[3], tri[4], tri[5]}, p2 = {tri[6], tri[7], tri[8]};
-    const v3 e1 = sub(p1, p0), e2 = sub(p2, p0);
+    return {p0, sub(p1, p0), sub(p2, p0)};
+}
+
+// Moller-Trumbore: t of the hit, or a negative value / NaN for none.
+__device__ __forceinline__ float ray_triangle(v3 o, v3 d, const Tri& tri) {
+    const v3 e1 = tri.e1, e2 = tri.e2;
     const v3 pv = cross(d, e2);
     const float det = dot(e1, pv);
     if (det == 0.0f) return -1.0f;
     const float inv = 1.0f / det;
-    const v3 s = sub(o, p0);
+    const v3 s = sub(o, tri.p0);
     const float u = dot(s, pv) * inv;
     if (u < 0.0f || u > 1.0f) return -1.0f;
     const v3 q = cross(s, e1);
@@ -147,7 +158,7 @@ __device__ __forceinline__ float nearest_hit(const LevelDev& L, uint32_t slot, c
     float best = INFINITY;
     for (uint32_t k = L.list_start[slot]; k < L.list_start[slot + 1]; ++k) {
         const uint32_t t = L.list[k];
-        const float th = ray_triangle(o, d, tris + (size_t)t * 9);
+        const float th = ray_triangle(o, d, load_tri(tris, t));
         if (th >= t_min && th < best) {
             best = th;
             tri_out = t;
@@ -228,22 +239,132 @@ __device__ __forceinline__ void onb(v3 n, v3& b1, v3& b2) {
 
 __device__ __forceinline__ float ray_eps(v3 o) { return kRayEps * (1.0f + sqrtf(dot(o, o))); }
 
-__global__ __launch_bounds__(kLabelThreads) void throughput_samples_kernel(
-    LevelsDev g, const float* __restrict__ tris, uint64_t seed, uint64_t first, uint32_t n, uint32_t spp,
-    uint32_t max_depth, uint64_t albedo_seed, float* __restrict__ inputs, float* __restrict__ targets,
-    float* __restrict__ valid) {
-    const uint32_t i = blockIdx.x * kLabelThreads + threadIdx.x;
-    if (i >= n) return;
-    uint64_t st = seed ^ ((first + i) * kGolden);
-    const uint32_t lod = index_draw(st, g.n_lods);
-    const LevelDev& L = g.l[lod];
-    const uint32_t slot = index_draw(st, L.n_occupied);
+// The n-th draw (n >= 1) after state s: the stream is a hash of a counter, so
+// the lanes of a group can evaluate the tries of a rejection loop side by side.
+__device__ __forceinline__ float uniform_at(uint64_t s, uint32_t n) {
+    s += (uint64_t)(n - 1) * kGolden;
+    return uniform01(s);
+}
+
+// ---- throughput samples
+//
+// A sample is a chain of spp paths (each continues the random stream where the
+// last one stopped), so it is the group of lanes given to one sample that has
+// to be fast.  G lanes share a sample: they split the voxel's triangle list in
+// every ray query, and evaluate the tries of a rejection loop at once.  The
+// list lengths of a pyramid differ by a factor of a hundred (blob mesh of 200k
+// triangles, 256^3 .. 16^3: means of 2, 3, 7, 23 and 105), so G follows the
+// sample's list: the smallest of 4, 16 and 64 whose lanes hold the list in
+// registers, kCached triangles each, for all paths of the sample; longer lists
+// run on 64 lanes and read their rest at every ray.  A block draws its samples' voxels,
+// sorts them by G and its waves take them from an LDS counter, 64 / G samples at
+// a time and the longest lists first.  What bounds it: VALU issue and, for few
+// samples, the chain of the slowest sample.  16384 samples of 64 paths of that
+// pyramid: 93.9 ms with one lane per sample (its wave waits for the longest
+// list, and 256 waves leave the chip idle), 1.50 ms like this.
+constexpr int kCached = 2;
+constexpr int kMaxBlockSamples = 64;
+
+struct SampleSetup {
+    uint64_t st;  // random stream after the draws below
+    uint32_t lod, slot, start, len;
+    v3 wo, wi;
+};
+
+// xor 1, xor 2 within a quad, then mirrors within 8 and 16 lanes: after the
+// steps for G lanes every lane of an aligned group has the group's result
+template <int G, typename T, typename Op>
+__device__ __forceinline__ T group_reduce(T v, Op op) {
+    static_assert(sizeof(T) == 4 && (G == 4 || G == 16 || G == 64), "");
+    auto dpp = [](T x, auto ctrl) {
+        return __builtin_bit_cast(
+            T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), decltype(ctrl)::value, 0xF, 0xF, false));
+    };
+    v = op(v, dpp(v, std::integral_constant<int, 0xB1>{}));
+    v = op(v, dpp(v, std::integral_constant<int, 0x4E>{}));
+    if constexpr (G >= 16) {
+        v = op(v, dpp(v, std::integral_constant<int, 0x141>{}));
+        v = op(v, dpp(v, std::integral_constant<int, 0x140>{}));
+    }
+    if constexpr (G == 64) {
+        v = op(v, __shfl_xor(v, 16, 64));
+        v = op(v, __shfl_xor(v, 32, 64));
+    }
+    return v;
+}
+
+// first lane (0 .. G-1) of the group whose flag is set, or G
+template <int G>
+__device__ __forceinline__ int group_first(bool flag, int lane) {
+    const uint64_t m = __ballot(flag);
+    if constexpr (G == 64) return m ? __builtin_ctzll(m) : G;
+    const uint32_t bits = (uint32_t)(m >> (lane & ~(G - 1))) & ((1u << (G & 31)) - 1u);
+    return bits ? __builtin_ctz(bits) : G;
+}
+
+template <int G>
+__device__ __forceinline__ v3 group_take(v3 v, int from, int lane) {
+    const int src = (lane & ~(G - 1)) + from;
+    return {__shfl(v.x, src, 64), __shfl(v.y, src, 64), __shfl(v.z, src, 64)};
+}
+
+// A voxel's triangle list spread over G lanes.
+template <int G>
+struct GroupList {
+    const float* tris;
+    const uint32_t* list;  // the voxel's entries
+    uint32_t len;
+    int sub;  // lane within the group
+    Tri tri[kCached];
+
+    __device__ __forceinline__ GroupList(const float* t, const uint32_t* l, uint32_t n, int lane_sub)
+        : tris(t), list(l), len(n), sub(lane_sub) {
+#pragma unroll
+        for (int r = 0; r < kCached; ++r) {
+            tri[r] = Tri{};  // no area: never hit
+            const uint32_t k = sub + r * G;
+            if (k < len) tri[r] = load_tri(tris, list[k]);
+        }
+    }
+
+    // Nearest hit with t >= t_min; the first in list order on ties.  Every lane gets it.
+    __device__ __forceinline__ float nearest(v3 o, v3 d, float t_min, uint32_t& entry) const {
+        float best = INFINITY;
+        uint32_t at = 0xffffffffu;
+        auto test = [&](const Tri& t, uint32_t k) {
+            const float th = ray_triangle(o, d, t);
+            if (th >= t_min && th < best) {
+                best = th;
+                at = k;
+            }
+        };
+#pragma unroll
+        for (int r = 0; r < kCached; ++r)
+            if (r == 0 || (uint32_t)(r * G) < len) test(tri[r], sub + r * G);
+        if (len > (uint32_t)(kCached * G)) {
+            for (uint32_t k = sub + kCached * G; k < len; k += G) test(load_tri(tris, list[k]), k);
+        }
+        best = best + 0.0f;  // -0 and +0 are one distance
+        const float all = group_reduce<G>(best, [](float a, float b) { return fminf(a, b); });
+        entry = group_reduce<G>(best == all ? at : 0xffffffffu, [](uint32_t a, uint32_t b) { return min(a, b); });
+        return all;
+    }
+};
+
+template <int G>
+__device__ __forceinline__ void throughput_sample(const LevelsDev& g, const float* __restrict__ tris,
+                                                  const SampleSetup& su, uint64_t i, uint32_t spp, uint32_t max_depth,
+                                                  uint64_t albedo_seed, float* __restrict__ inputs,
+                                                  float* __restrict__ targets, float* __restrict__ valid) {
+    const int lane = threadIdx.x & 63, sub = lane & (G - 1);
+    const LevelDev& L = g.l[su.lod];
+    uint64_t st = su.st;
     uint32_t vx, vy, vz;
-    voxel_xyz(L.occupied[slot], L.res, vx, vy, vz);
-    const v3 wo = sphere_dir(st);
-    const v3 wi = sphere_dir(st);
+    voxel_xyz(L.occupied[su.slot], L.res, vx, vy, vz);
+    const v3 wo = su.wo, wi = su.wi;
     const Box box = voxel_box(g, L, vx, vy, vz);
     const float U = fmaxf(L.unit[0], fmaxf(L.unit[1], L.unit[2]));
+    const GroupList<G> list(tris, L.list + su.start, su.len, sub);
     v3 u_ax, v_ax;
     onb(wo, u_ax, v_ax);
     const v3 d0 = {-wo.x, -wo.y, -wo.z};
@@ -251,12 +372,13 @@ __global__ __launch_bounds__(kLabelThreads) void throughput_samples_kernel(
     v3 sum = {0.0f, 0.0f, 0.0f};
     uint32_t n_valid = 0;
     for (uint32_t j = 0; j < spp; ++j) {
-        // entry point: offsets on the plane through centre + 2U wo, normal wo
+        // entry point: offsets on the plane through centre + 2U wo, normal wo;
+        // lane `sub` evaluates try base + sub
         bool found = false;
         v3 entry = box.c;
-        for (int k = 0; k < kMaxDraws && !found; ++k) {
-            const float ox = (uniform01(st) * 2.0f - 1.0f) * U;
-            const float oy = (uniform01(st) * 2.0f - 1.0f) * U;
+        for (int base = 0; base < kMaxDraws && !found; base += G) {
+            const float ox = (uniform_at(st, 2 * (base + sub) + 1) * 2.0f - 1.0f) * U;
+            const float oy = (uniform_at(st, 2 * (base + sub) + 2) * 2.0f - 1.0f) * U;
             const v3 o = {((box.c.x + wo.x * back) + u_ax.x * ox) + v_ax.x * oy,
                           ((box.c.y + wo.y * back) + u_ax.y * ox) + v_ax.y * oy,
                           ((box.c.z + wo.z * back) + u_ax.z * ox) + v_ax.z * oy};
@@ -264,6 +386,7 @@ __global__ __launch_bounds__(kLabelThreads) void throughput_samples_kernel(
             bool miss = false;
             const float oc[3] = {o.x, o.y, o.z}, dc[3] = {d0.x, d0.y, d0.z};
             const float lo[3] = {box.lo.x, box.lo.y, box.lo.z}, hi[3] = {box.hi.x, box.hi.y, box.hi.z};
+#pragma unroll
             for (int a = 0; a < 3; ++a) {
                 if (dc[a] == 0.0f) {
                     if (oc[a] < lo[a] || oc[a] > hi[a]) miss = true;
@@ -274,26 +397,30 @@ __global__ __launch_bounds__(kLabelThreads) void throughput_samples_kernel(
                 if (t0 > tn) tn = t0;
                 if (t1 < tf) tf = t1;
             }
-            if (!miss && tn <= tf && tf >= 0.0f) {
-                entry = along(o, tn, d0);
-                found = true;
+            const int first = group_first<G>(!miss && tn <= tf && tf >= 0.0f, lane);
+            found = first < G;
+            if (found) {
+                entry = group_take<G>(along(o, tn, d0), first, lane);
+                st += (uint64_t)(2 * (base + first + 1)) * kGolden;
             }
         }
-        if (!found) continue;
+        if (!found) {
+            st += (uint64_t)(2 * kMaxDraws) * kGolden;
+            continue;
+        }
         v3 o = entry, d = d0, T = {1.0f, 1.0f, 1.0f}, acc = {0.0f, 0.0f, 0.0f};
         float t_min = 0.0f;
         bool path_valid = false;
         for (uint32_t bounce = 0; bounce < max_depth; ++bounce) {
-            uint32_t tri = 0;
-            const float t = nearest_hit(L, slot, tris, o, d, t_min, tri);
+            uint32_t at = 0;
+            const float t = list.nearest(o, d, t_min, at);
             if (!(t < INFINITY)) break;
             const v3 p = along(o, t, d);
             if (!in_box(box, p)) break;
             if (bounce == 0) path_valid = true;
-            const float* tv = tris + (size_t)tri * 9;
-            const v3 e1 = {tv[3] - tv[0], tv[4] - tv[1], tv[5] - tv[2]};
-            const v3 e2 = {tv[6] - tv[0], tv[7] - tv[1], tv[8] - tv[2]};
-            v3 nrm = cross(e1, e2);
+            const uint32_t tri = list.list[at];
+            const Tri tv = load_tri(tris, tri);
+            v3 nrm = cross(tv.e1, tv.e2);
             const float inv_len = 1.0f / sqrtf(dot(nrm, nrm));
             nrm = {nrm.x * inv_len, nrm.y * inv_len, nrm.z * inv_len};
             const v3 wout = {-d.x, -d.y, -d.z};
@@ -304,7 +431,7 @@ __global__ __launch_bounds__(kLabelThreads) void throughput_samples_kernel(
             const float cos_i = dot(wi, nrm);
             if (cos_i > 0.0f) {
                 uint32_t t2i = 0;
-                const float t2 = nearest_hit(L, slot, tris, p, wi, eps, t2i);
+                const float t2 = list.nearest(p, wi, eps, t2i);
                 if (!(t2 < INFINITY) || !in_box(box, along(p, t2, wi))) {
                     acc.x = acc.x + (T.x * (alb.x * kInvPi)) * cos_i;
                     acc.y = acc.y + (T.y * (alb.y * kInvPi)) * cos_i;
@@ -313,14 +440,20 @@ __global__ __launch_bounds__(kLabelThreads) void throughput_samples_kernel(
             }
             // cosine-weighted continuation: uniform disk point lifted to the hemisphere
             float x = 0.0f, y = 0.0f;
-            for (int k = 0; k < kMaxDraws; ++k) {
-                const float x1 = uniform01(st) * 2.0f - 1.0f, y1 = uniform01(st) * 2.0f - 1.0f;
-                if (x1 * x1 + y1 * y1 <= 1.0f) {
-                    x = x1;
-                    y = y1;
-                    break;
+            bool in_disk = false;
+            for (int base = 0; base < kMaxDraws && !in_disk; base += G) {
+                const float x1 = uniform_at(st, 2 * (base + sub) + 1) * 2.0f - 1.0f;
+                const float y1 = uniform_at(st, 2 * (base + sub) + 2) * 2.0f - 1.0f;
+                const int first = group_first<G>(x1 * x1 + y1 * y1 <= 1.0f, lane);
+                in_disk = first < G;
+                if (in_disk) {
+                    const v3 xy = group_take<G>({x1, y1, 0.0f}, first, lane);
+                    x = xy.x;
+                    y = xy.y;
+                    st += (uint64_t)(2 * (base + first + 1)) * kGolden;
                 }
             }
+            if (!in_disk) st += (uint64_t)(2 * kMaxDraws) * kGolden;
             const float zz = sqrtf(fmaxf(0.0f, 1.0f - (x * x + y * y)));
             v3 b1, b2;
             onb(nrm, b1, b2);
@@ -335,23 +468,91 @@ __global__ __launch_bounds__(kLabelThreads) void throughput_samples_kernel(
             ++n_valid;
         }
     }
-    float* in = inputs + (size_t)i * 10;
-    in[0] = (box.c.x - g.bmin[0]) / (g.bmax[0] - g.bmin[0]);
-    in[1] = (box.c.y - g.bmin[1]) / (g.bmax[1] - g.bmin[1]);
-    in[2] = (box.c.z - g.bmin[2]) / (g.bmax[2] - g.bmin[2]);
-    in[3] = (wo.x + 1.0f) * 0.5f;
-    in[4] = (wo.y + 1.0f) * 0.5f;
-    in[5] = (wo.z + 1.0f) * 0.5f;
-    in[6] = (wi.x + 1.0f) * 0.5f;
-    in[7] = (wi.y + 1.0f) * 0.5f;
-    in[8] = (wi.z + 1.0f) * 0.5f;
-    in[9] = (float)lod;
-    const float nv = (float)n_valid;
-    float* out = targets + (size_t)i * 3;
-    out[0] = n_valid ? sum.x / nv : 0.0f;
-    out[1] = n_valid ? sum.y / nv : 0.0f;
-    out[2] = n_valid ? sum.z / nv : 0.0f;
-    valid[i] = n_valid ? 1.0f : 0.0f;
+    if (sub == 0) {
+        float* in = inputs + i * 10;
+        in[0] = (box.c.x - g.bmin[0]) / (g.bmax[0] - g.bmin[0]);
+        in[1] = (box.c.y - g.bmin[1]) / (g.bmax[1] - g.bmin[1]);
+        in[2] = (box.c.z - g.bmin[2]) / (g.bmax[2] - g.bmin[2]);
+        in[3] = (wo.x + 1.0f) * 0.5f;
+        in[4] = (wo.y + 1.0f) * 0.5f;
+        in[5] = (wo.z + 1.0f) * 0.5f;
+        in[6] = (wi.x + 1.0f) * 0.5f;
+        in[7] = (wi.y + 1.0f) * 0.5f;
+        in[8] = (wi.z + 1.0f) * 0.5f;
+        in[9] = (float)su.lod;
+        const float nv = (float)n_valid;
+        float* out = targets + i * 3;
+        out[0] = n_valid ? sum.x / nv : 0.0f;
+        out[1] = n_valid ? sum.y / nv : 0.0f;
+        out[2] = n_valid ? sum.z / nv : 0.0f;
+        valid[i] = n_valid ? 1.0f : 0.0f;
+    }
+}
+
+__global__ __launch_bounds__(kLabelThreads, 4) void throughput_samples_kernel(
+    LevelsDev g, const float* __restrict__ tris, uint64_t seed, uint64_t first, uint32_t n, uint32_t block_samples,
+    uint32_t spp, uint32_t max_depth, uint64_t albedo_seed, float* __restrict__ inputs, float* __restrict__ targets,
+    float* __restrict__ valid) {
+    __shared__ SampleSetup setup[kMaxBlockSamples];
+    __shared__ uint8_t order[kMaxBlockSamples];  // samples on 64 lanes, then on 16, then on 4
+    __shared__ uint32_t n_of[3];
+    __shared__ uint32_t next_item;
+    const uint64_t i0 = (uint64_t)blockIdx.x * block_samples;
+    const int lane = threadIdx.x & 63;
+    if (threadIdx.x < 64) {
+        const bool mine = (uint32_t)lane < block_samples && i0 + lane < n;
+        uint32_t len = 0;
+        if (mine) {
+            SampleSetup su;
+            su.st = seed ^ ((first + i0 + lane) * kGolden);
+            su.lod = index_draw(su.st, g.n_lods);
+            const LevelDev& L = g.l[su.lod];
+            su.slot = index_draw(su.st, L.n_occupied);
+            su.wo = sphere_dir(su.st);
+            su.wi = sphere_dir(su.st);
+            su.start = L.list_start[su.slot];
+            su.len = len = L.list_start[su.slot + 1] - su.start;
+            setup[lane] = su;
+        }
+        const uint64_t below = (1ull << lane) - 1;
+        const int cls = len > 16 * kCached ? 0 : len > 4 * kCached ? 1 : 2;
+        uint32_t at = 0;
+        for (int c = 0; c < 3; ++c) {
+            const uint64_t m = __ballot(mine && cls == c);
+            if (mine && cls == c) order[at + __popcll(m & below)] = (uint8_t)lane;
+            at += (uint32_t)__popcll(m);
+            if (lane == 0) n_of[c] = (uint32_t)__popcll(m);
+        }
+        if (lane == 0) next_item = 0;
+    }
+    __syncthreads();
+    const uint32_t n64 = n_of[0], n16 = n_of[1], n4 = n_of[2];
+    const uint32_t items16 = (n16 + 3) / 4, items4 = (n4 + 15) / 16;
+    for (;;) {
+        // every lane counts, so an item is 64: a branch on the lane here would be
+        // threaded with the one that ends a sample, and lanes would go on alone
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t item = (uint32_t)__builtin_amdgcn_readfirstlane((int)atomicAdd(&next_item, 1u)) / 64u;
+        if (item >= n64 + items16 + items4) break;
+        if (item < n64) {
+            const uint32_t sm = order[item];
+            throughput_sample<64>(g, tris, setup[sm], i0 + sm, spp, max_depth, albedo_seed, inputs, targets, valid);
+        } else if (item < n64 + items16) {
+            const uint32_t k = (item - n64) * 4 + lane / 16;
+            if (k < n16) {
+                const uint32_t sm = order[n64 + k];
+                throughput_sample<16>(g, tris, setup[sm], i0 + sm, spp, max_depth, albedo_seed, inputs, targets,
+                                      valid);
+            }
+        } else {
+            const uint32_t k = (item - n64 - items16) * 16 + lane / 4;
+            if (k < n4) {
+                const uint32_t sm = order[n64 + n16 + k];
+                throughput_sample<4>(g, tris, setup[sm], i0 + sm, spp, max_depth, albedo_seed, inputs, targets,
+                                     valid);
+            }
+        }
+    }
 }
 
 // glm min(x, y) = (y < x) ? y : x, max(x, y) = (x < y) ? y : x
@@ -498,9 +699,15 @@ void labeler_throughput(const Labeler& lb, hipStream_t s, uint64_t seed, uint64_
     NLOD_CHECK(inputs != nullptr && targets != nullptr && valid != nullptr, "output pointers are null");
     NLOD_CHECK(spp >= 1 && spp <= 4096, "spp must be in [1, 4096]");
     NLOD_CHECK(max_depth >= 1 && max_depth <= 64, "max_depth must be in [1, 64]");
-    hipLaunchKernelGGL(throughput_samples_kernel, dim3(div_round_up(n, kLabelThreads)), dim3(kLabelThreads), 0, s,
-                       lb.device_view(), lb.d_tris, seed, first, n, spp, max_depth, albedo_seed, inputs, targets,
-                       valid);
+    // samples per block: enough blocks for every CU to hold four, and no more
+    // samples than that takes, since a block's waves fill up better with more
+    uint32_t block_samples = 4;
+    while (block_samples < (uint32_t)kMaxBlockSamples &&
+           (uint64_t)block_samples * 4 * (uint64_t)cu_count() < n)
+        block_samples *= 2;
+    hipLaunchKernelGGL(throughput_samples_kernel, dim3(div_round_up(n, block_samples)), dim3(kLabelThreads), 0, s,
+                       lb.device_view(), lb.d_tris, seed, first, n, block_samples, spp, max_depth, albedo_seed,
+                       inputs, targets, valid);
     NLOD_LAUNCH_CHECK();
 }
 

@@ -76,6 +76,26 @@ def test_throughput_matches_oracle(oracle, cuda, n_lods):
     assert 0 < ev.mean() < 1 and et.max() > 0
 
 
+@pytest.mark.parametrize("n,spp,max_depth", [(1, 5, 3), (5, 1, 1), (63, 3, 9), (4097, 2, 2)])
+def test_throughput_block_edges(oracle, cuda, n, spp, max_depth):
+    """Blocks that are not full, on lists of every group width: 4 lanes (up to 8
+    triangles), 16 (up to 32), 64, and 64 with triangles beyond the 128 kept in
+    registers.  The stream, and so every bit, is the oracle's."""
+    from neural_lod_amd.labels import Labeler
+    tris = S.blob_mesh(20_000, seed=6)
+    print(f"case throughput edges n={n} spp={spp} depth={max_depth}", flush=True)
+    lb = Labeler(torch.from_numpy(tris).cuda(), 64, 4)
+    longest = [lv["n_list_entries"] / lv["n_occupied"] for lv in lb.levels]
+    assert longest[0] < 8 and longest[-1] > 64  # short and long lists both occur
+    x, t, v = lb.throughput(n, seed=3, first=10 ** 9, spp=spp, max_depth=max_depth, albedo_seed=8)
+    torch.cuda.synchronize()
+    ex, et, ev, _ = oracle.throughput_samples(tris, 64, 4, seed=3, first=10 ** 9, n=n, spp=spp, max_depth=max_depth,
+                                              albedo_seed=8)
+    assert np.array_equal(x.cpu().numpy(), ex)
+    assert np.array_equal(v.cpu().numpy(), ev)
+    assert np.array_equal(t.cpu().numpy(), et), f"{int((t.cpu().numpy() != et).any(axis=1).sum())} targets differ"
+
+
 def test_throughput_invalid_arguments(cuda):
     from neural_lod_amd._lib import NlodError
     from neural_lod_amd.labels import Labeler
