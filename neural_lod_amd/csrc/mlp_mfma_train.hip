@@ -11,9 +11,9 @@
 // accumulator layout, then G_{l-1} = W_l^T delta_l on MFMA with the transposed
 // weights pre-packed (columns permuted to the accumulator layout of delta_l),
 // delta_{l-1} = G_{l-1} * act'(H_{l-1}); finally dL/d(enc) = W_0^T delta_0.
-// Weight gradients dW_l = sum_q delta_l[u][q] H_{l-1}[k][q] use
-// v_mfma_f32_16x16x16_f16 with the queries as the reduction dimension, split
-// over query chunks with a deterministic second-pass reduction.
+// Weight gradients dW_l = sum_q delta_l[u][q] H_{l-1}[k][q] have the queries as
+// the reduction dimension, split over query chunks with a deterministic
+// second-pass reduction.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -22,21 +22,15 @@
 #include "mfma_common.h"
 #include "model.h"
 #include "nlod_common.h"
+#include "wgrad.h"
 
 namespace nlod {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr uint32_t kWgradTilesPerBlock = 64;  // 1024 queries per weight-gradient partial
-
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ size_t unit_major(uint32_t tile, uint32_t units, uint32_t u, uint32_t n) {
     return ((size_t)tile * units + u) * 16 + n;
-}
-
-__device__ __forceinline__ floatx4 mfma16x16x16(const half4_t& a, const half4_t& b, const floatx4& c) {
-    return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
 }
 
 struct TrainArgs {
@@ -212,82 +206,110 @@ __global__ __launch_bounds__(kBlock) void mlp_bwd_kernel(TrainArgs a, const half
     }
 }
 
-// dW partials: grid (chunks, L+1).  Matrix l: rows = units of layer l's output
-// (16 for the output layer), cols = inputs (K for layer 0).  Wave w of a block
-// owns output tiles t = w, w+4, ... of the matrix and reduces over the chunk's
-// query tiles.
-template <int W>
-__global__ __launch_bounds__(kBlock) void wgrad_mfma_kernel(TrainArgs a, const half_t* __restrict__ feat,
-                                                            const half_t* __restrict__ H,
-                                                            const half_t* __restrict__ D,
-                                                            float* __restrict__ partial, uint32_t partial_stride) {
-    constexpr int MAXT = (W / 16) * (W / 16) / 4 > 0 ? (W / 16) * (W / 16) / 4 : 1;
-    constexpr int TPW = MAXT < 1 ? 1 : MAXT;  // tiles per wave upper bound for hidden layers
+// dW partials: grid (chunks, 64 x 64 tiles of all matrices), see wgrad.h.  The
+// reduction dimension is the queries: one v_mfma_f32_16x16x32_f16 takes 32 of
+// them, lane group g the 8 queries 8 (g & 1) of query tile 2 step + (g >> 1), so
+// a fragment of the unit-major tensors is one 16-byte load a lane.  The next
+// step's fragments load while the current step's MFMAs run.
+// 101003 queries through the 144-input 128 x 4 network: one block per (1024
+// queries, matrix), whose waves loaded two fragments per 16x16x16 MFMA, took
+// 931 us of a 1.46 ms training step, which is 0.58 ms with this split.
+template <int RT, int CT>
+__device__ __forceinline__ void wgrad_tile(const TrainArgs& a, const WgradItem& it, uint32_t step0, uint32_t step1,
+                                           const half_t* __restrict__ feat, const half_t* __restrict__ Hp,
+                                           const half_t* __restrict__ Dl, uint32_t d_units, float* __restrict__ p,
+                                           uint32_t ld, float4* lds) {
     const int lane = threadIdx.x & 63, g = lane >> 4, m16 = lane & 15, wave = threadIdx.x >> 6;
-    const uint32_t L = a.n_hidden_layers;
-    const uint32_t layer = blockIdx.y;  // 0 .. L
-    const uint32_t n_tiles = (a.N + 15) / 16;
-    const size_t layer_stride = (size_t)n_tiles * W * 16;
-    const uint32_t rows = layer == L ? 16u : (uint32_t)W;
-    const uint32_t cols = layer == 0 ? a.k_padded : (uint32_t)W;
-    const uint32_t rt = rows / 16, ct = cols / 16, n_out_tiles = rt * ct;
-    const uint32_t kp2 = a.k_padded / 2;
-    const half_t* Dl = D + (size_t)layer * layer_stride;  // layer L: the output deltas
-    const uint32_t d_units = layer == L ? 16u : (uint32_t)W;
-    const half_t* Hp = layer == 0 ? nullptr : H + (size_t)(layer - 1) * layer_stride;
-    // up to 4 * TPW output tiles per block pass; loop if the matrix has more (layer 0 with a wide K)
-    for (uint32_t t0 = 0; t0 < n_out_tiles; t0 += 4 * TPW) {
-        floatx4 acc[TPW];
+    const uint32_t n_tiles = (a.N + 15) / 16, W = a.width, kp2 = a.k_padded / 2;
+    floatx4 acc[RT * CT];
 #pragma unroll
-        for (int t = 0; t < TPW; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-        const uint32_t tile_begin = blockIdx.x * kWgradTilesPerBlock;
-        const uint32_t tile_end = min(n_tiles, tile_begin + kWgradTilesPerBlock);
-        for (uint32_t qt = tile_begin; qt < tile_end; ++qt) {
+    for (int t = 0; t < RT * CT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const uint32_t half_sel = (m16 & 1) ? 0x07060302u : 0x05040100u;
+    auto load = [&](uint32_t step, half8 (&d)[RT], half8 (&x)[CT]) {
+        const uint32_t qt = 2 * step + (uint32_t)(g >> 1), q8 = 8u * (uint32_t)(g & 1);
+        const uint32_t tile = min(qt, n_tiles - 1);
 #pragma unroll
-            for (int t = 0; t < TPW; ++t) {
-                const uint32_t ot = t0 + (uint32_t)wave + 4u * (uint32_t)t;
-                if (ot >= n_out_tiles) break;
-                const uint32_t mr = ot / ct, nc = ot % ct;
-                // A = delta[u = 16 mr + m16][q = 4g..4g+3]
-                const half4_t av = *reinterpret_cast<const half4_t*>(Dl + unit_major(qt, d_units, 16 * mr + m16, 4 * g));
-                half4_t bv;
-                const uint32_t k = 16 * nc + m16;
-                if (layer == 0) {  // B = X[k][q], X in the pair layout
-                    const half_t* fb = feat + feat_pair_offset(qt, k >> 1, kp2, 0) + (k & 1);
+        for (int r = 0; r < RT; ++r)
+            d[r] = *reinterpret_cast<const half8*>(Dl + unit_major(tile, d_units, it.row0 + 16 * r + m16, q8));
+        if (it.layer == 0) {  // X in the pair layout: this lane's half of 8 queries' pairs
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) bv[j] = fb[(4 * g + j) * 2];
-                } else {
-                    bv = *reinterpret_cast<const half4_t*>(Hp + unit_major(qt, W, k, 4 * g));
-                }
-                acc[t] = mfma16x16x16(av, bv, acc[t]);
+            for (int c = 0; c < CT; ++c) {
+                const uint32_t k = it.col0 + 16 * c + m16;
+                const uint4* w = reinterpret_cast<const uint4*>(feat + feat_pair_offset(tile, k >> 1, kp2, q8));
+                const uint4 w0 = w[0], w1 = w[1];
+                const uint4 v = {__builtin_amdgcn_perm(w0.y, w0.x, half_sel), __builtin_amdgcn_perm(w0.w, w0.z, half_sel),
+                                 __builtin_amdgcn_perm(w1.y, w1.x, half_sel), __builtin_amdgcn_perm(w1.w, w1.z, half_sel)};
+                x[c] = __builtin_bit_cast(half8, v);
             }
-        }
-        // write this chunk's partial (row-major [rows][cols] of the matrix)
-        float* p = partial + (size_t)blockIdx.x * partial_stride;
-        const size_t moff = layer == 0 ? 0 : (size_t)W * a.k_enc + (size_t)(layer - 1) * W * W;
-        const uint32_t ld = layer == 0 ? a.k_enc : (uint32_t)W;
+        } else {
 #pragma unroll
-        for (int t = 0; t < TPW; ++t) {
-            const uint32_t ot = t0 + (uint32_t)wave + 4u * (uint32_t)t;
-            if (ot >= n_out_tiles) break;
-            const uint32_t mr = ot / ct, nc = ot % ct;
+            for (int c = 0; c < CT; ++c)
+                x[c] = *reinterpret_cast<const half8*>(Hp + unit_major(tile, W, it.col0 + 16 * c + m16, q8));
+        }
+        if (2 * step + 1 >= n_tiles) {  // the last step of an odd number of query tiles
+            const half8 zero = {};
+#pragma unroll
+            for (int r = 0; r < RT; ++r) d[r] = qt < n_tiles ? d[r] : zero;
+#pragma unroll
+            for (int c = 0; c < CT; ++c) x[c] = qt < n_tiles ? x[c] : zero;
+        }
+    };
+    half8 nd[RT], nx[CT];
+    uint32_t step = step0 + (uint32_t)wave;
+    if (step < step1) load(step, nd, nx);
+    for (; step < step1; step += 4) {
+        half8 d[RT], x[CT];
+#pragma unroll
+        for (int r = 0; r < RT; ++r) d[r] = nd[r];
+#pragma unroll
+        for (int c = 0; c < CT; ++c) x[c] = nx[c];
+        if (step + 4 < step1) load(step + 4, nd, nx);
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) acc[r * CT + c] = mfma16(d[r], x[c], acc[r * CT + c]);
+    }
+    wgrad_add_waves<RT * CT>(acc, lds);
+    if (wave != 0) return;
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const uint32_t r = 16 * mr + 4 * g + i, c = 16 * nc + m16;
-                if (c < ld) p[moff + (size_t)r * ld + c] = acc[t][i];
+                const uint32_t row = it.row0 + 16 * r + 4 * g + i, col = it.col0 + 16 * c + m16;
+                if (col < ld) p[(size_t)row * ld + col] = acc[r * CT + c][i];
             }
-        }
-    }
 }
 
-__global__ __launch_bounds__(256) void wgrad_reduce_kernel(uint32_t n_elems, uint32_t n_chunks, uint32_t stride,
-                                                           const float* __restrict__ partial, float* __restrict__ out,
-                                                           int accumulate) {
-    const uint32_t e = blockIdx.x * 256 + threadIdx.x;
-    if (e >= n_elems) return;
-    float s = 0.0f;
-    for (uint32_t c = 0; c < n_chunks; ++c) s += partial[(size_t)c * stride + e];
-    out[e] = accumulate ? out[e] + s : s;
+__global__ __launch_bounds__(kBlock, 3) void wgrad_mfma_kernel(TrainArgs a, const half_t* __restrict__ feat,
+                                                               const half_t* __restrict__ H,
+                                                               const half_t* __restrict__ D,
+                                                               float* __restrict__ partial, uint32_t partial_stride,
+                                                               uint32_t chunk_steps) {
+    __shared__ float4 lds[2 * 16 * 64];
+    const uint32_t L = a.n_hidden_layers, W = a.width;
+    const WgradItem it = wgrad_item(blockIdx.y, WgradShape{W, a.k_padded, L, 16});
+    const uint32_t n_tiles = (a.N + 15) / 16, n_steps = (n_tiles + 1) / 2;
+    const uint32_t step0 = min(n_steps, blockIdx.x * chunk_steps), step1 = min(n_steps, step0 + chunk_steps);
+    const size_t layer_stride = (size_t)n_tiles * W * 16;
+    const uint32_t rows = it.layer == L ? 16u : W, cols = it.layer == 0 ? a.k_padded : W;
+    const uint32_t ld = it.layer == 0 ? a.k_enc : W;
+    const half_t* Dl = D + (size_t)it.layer * layer_stride;  // layer L: the output deltas
+    const half_t* Hp = it.layer == 0 ? nullptr : H + (size_t)(it.layer - 1) * layer_stride;
+    float* p = partial + (size_t)blockIdx.x * partial_stride +
+               (it.layer == 0 ? 0 : (size_t)W * a.k_enc + (size_t)(it.layer - 1) * W * W);
+    auto run = [&](auto RTc, auto CTc) {
+        wgrad_tile<decltype(RTc)::value, decltype(CTc)::value>(a, it, step0, step1, feat, Hp, Dl, rows, p, ld, lds);
+    };
+    auto run_rows = [&](auto RTc) {  // widths are multiples of 32, so a tile is 32 or 64 wide
+        if (cols - it.col0 >= kWgradTile) run(RTc, std::integral_constant<int, 4>{});
+        else run(RTc, std::integral_constant<int, 2>{});
+    };
+    const uint32_t rt = (rows - it.row0) / 16;
+    if (rt >= 4) run_rows(std::integral_constant<int, 4>{});
+    else if (rt >= 2) run_rows(std::integral_constant<int, 2>{});
+    else run_rows(std::integral_constant<int, 1>{});
 }
 
 TrainArgs make_targs(const Layout& L, uint32_t N) {
@@ -362,9 +384,13 @@ void mfma_mlp_backward(hipStream_t stream, const Layout& L, const void* packed_b
     NLOD_LAUNCH_CHECK();
 }
 
+static uint32_t wgrad_steps(uint32_t N) { return div_round_up(div_round_up(std::max<uint32_t>(N, 1), 16), 2); }
+static uint32_t wgrad_chunks_of(const Layout& L, uint32_t N) {
+    return wgrad_chunks(wgrad_items({L.net.width, k_padded_of(L.net), L.net.n_hidden_layers, 16}), wgrad_steps(N));
+}
+
 size_t mfma_wgrad_workspace_floats(const Layout& L, uint32_t N) {
-    const uint32_t chunks = div_round_up(div_round_up(std::max<uint32_t>(N, 1), 16), kWgradTilesPerBlock);
-    return (size_t)chunks * L.net.n_params();
+    return (size_t)wgrad_chunks_of(L, N) * L.net.n_params();
 }
 
 void mfma_weight_grad(hipStream_t stream, const Layout& L, const void* feat, const void* hidden, const void* delta,
@@ -376,17 +402,13 @@ void mfma_weight_grad(hipStream_t stream, const Layout& L, const void* feat, con
         return;
     }
     const TrainArgs a = make_targs(L, N);
-    const uint32_t chunks = div_round_up(div_round_up(N, 16), kWgradTilesPerBlock);
-    by_w(L.net.width, [&](auto Wc) {
-        constexpr int W = decltype(Wc)::value;
-        hipLaunchKernelGGL(wgrad_mfma_kernel<W>, dim3(chunks, L.net.n_hidden_layers + 1), dim3(kBlock), 0, stream, a,
-                           static_cast<const half_t*>(feat), static_cast<const half_t*>(hidden),
-                           static_cast<const half_t*>(delta), workspace, n_net);
-    });
+    const uint32_t chunks = wgrad_chunks_of(L, N);
+    const uint32_t items = wgrad_items({a.width, a.k_padded, a.n_hidden_layers, 16});
+    hipLaunchKernelGGL(wgrad_mfma_kernel, dim3(chunks, items), dim3(kBlock), 0, stream, a,
+                       static_cast<const half_t*>(feat), static_cast<const half_t*>(hidden),
+                       static_cast<const half_t*>(delta), workspace, n_net, div_round_up(wgrad_steps(N), chunks));
     NLOD_LAUNCH_CHECK();
-    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(div_round_up(n_net, 256)), dim3(256), 0, stream, n_net, chunks, n_net,
-                       workspace, grads, accumulate ? 1 : 0);
-    NLOD_LAUNCH_CHECK();
+    partial_reduce(stream, n_net, chunks, workspace, grads, accumulate);
 }
 
 }  // namespace nlod
