@@ -64,6 +64,20 @@ inline size_t packed_halves(const NetShape& n) {
     return frags * 64 * 8;
 }
 
+// Copies packed weights (whole fragments, so a multiple of 512 halves) into LDS
+// with direct-to-LDS loads: a block of NT threads has all of them in flight at
+// once, without registers (a copy loop waits for each load: several microseconds
+// for the 143 KB of a 128-wide network).  The caller synchronizes the block.
+template <int NT>
+__device__ __forceinline__ void stage_weights(half_t* lds, const half_t* __restrict__ src, uint32_t halves) {
+    typedef const __attribute__((address_space(1))) void* global_ptr;
+    typedef __attribute__((address_space(3))) void* lds_ptr;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63u;
+    for (uint32_t k = wave * 512; k < halves; k += NT * 8)
+        __builtin_amdgcn_global_load_lds((global_ptr)(src + k + lane * 8), (lds_ptr)(lds + k), 16, 0, 0);
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's copies have landed
+}
+
 // k-slot (g, j) of chunk c of a layer fed by the previous layer's accumulators
 // -> hidden unit: slots 0-3 come from accumulator tile 2c, 4-7 from tile 2c+1.
 __host__ __device__ inline uint32_t permuted_unit(uint32_t c, uint32_t g, uint32_t j) {

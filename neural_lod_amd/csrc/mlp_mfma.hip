@@ -265,23 +265,23 @@ struct MlpArgs16 {
 // compile time, and each wave loads the feature fragments of its next group
 // while it computes the current one (the loads are then in flight for a whole
 // group's MFMAs); KC0 = 0: width from the arguments, loaded as used.
-template <int W, int TT, int ACT, int KC0>
-__global__ __launch_bounds__(kBlock) void mlp_fwd_kernel(MlpArgs16 a, const half_t* __restrict__ packed,
+// NT: threads per block (see mfma_mlp_forward).
+template <int W, int TT, int ACT, int KC0, int NT>
+__global__ __launch_bounds__(NT) void mlp_fwd_kernel(MlpArgs16 a, const half_t* __restrict__ packed,
                                                          const half_t* __restrict__ feat, float* __restrict__ out) {
     constexpr int MT = W / 16, KC = W / 32;
     constexpr int PF = KC0 > 0 ? KC0 : 1;
     const int act = ACT >= 0 ? ACT : a.act;
     extern __shared__ float4 smem4[];
     half_t* sw = reinterpret_cast<half_t*>(smem4);
-    for (uint32_t k = threadIdx.x; k < a.packed_halves / 8; k += kBlock)
-        reinterpret_cast<float4*>(sw)[k] = reinterpret_cast<const float4*>(packed)[k];
+    stage_weights<NT>(sw, packed, a.packed_halves);
     __syncthreads();
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
     const uint32_t kc0 = KC0 > 0 ? (uint32_t)KC0 : a.k_padded / 32, kp2 = a.k_padded / 2;
     const uint32_t n_tiles = (a.N + 15) / 16;
     const uint32_t n_groups = (n_tiles + TT - 1) / TT;
-    const uint32_t n_waves = gridDim.x * (kBlock / 64);
-    const uint32_t grp0 = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+    const uint32_t n_waves = gridDim.x * (NT / 64);
+    const uint32_t grp0 = blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
     half8 nb[TT][PF];  // KC0 > 0: fragments of the wave's next group
     auto load_group = [&](uint32_t gi) {
 #pragma unroll
@@ -380,17 +380,22 @@ __global__ __launch_bounds__(kBlock) void mlp_fwd_kernel(MlpArgs16 a, const half
     }
 }
 
-// ReLU networks with inputs up to 128 features take the prefetching kernels
-template <int W, int TT, typename Launch>
+// ReLU networks with inputs up to 128 features (32 at width 128, where more
+// prefetched fragments would spill) take the prefetching kernels
+template <int W, int TT, int NT, typename Launch>
 void launch_fwd(const MlpArgs16& a, Launch&& launch) {
-    if (a.act != ACT_RELU) return launch(mlp_fwd_kernel<W, TT, -1, 0>, TT);
-    switch (a.k_padded / 32) {
-        case 1: return launch(mlp_fwd_kernel<W, TT, ACT_RELU, 1>, TT);
-        case 2: return launch(mlp_fwd_kernel<W, TT, ACT_RELU, 2>, TT);
-        case 3: return launch(mlp_fwd_kernel<W, TT, ACT_RELU, 3>, TT);
-        case 4: return launch(mlp_fwd_kernel<W, TT, ACT_RELU, 4>, TT);
-        default: return launch(mlp_fwd_kernel<W, TT, ACT_RELU, 0>, TT);
+    if (a.act != ACT_RELU) return launch(mlp_fwd_kernel<W, TT, -1, 0, NT>, TT, NT);
+    const uint32_t kc = a.k_padded / 32;
+    if (kc == 1) return launch(mlp_fwd_kernel<W, TT, ACT_RELU, 1, NT>, TT, NT);
+    if constexpr (W < 128) {
+        switch (kc) {
+            case 2: return launch(mlp_fwd_kernel<W, TT, ACT_RELU, 2, NT>, TT, NT);
+            case 3: return launch(mlp_fwd_kernel<W, TT, ACT_RELU, 3, NT>, TT, NT);
+            case 4: return launch(mlp_fwd_kernel<W, TT, ACT_RELU, 4, NT>, TT, NT);
+            default: break;
+        }
     }
+    launch(mlp_fwd_kernel<W, TT, ACT_RELU, 0, NT>, TT, NT);
 }
 
 __global__ void to_half_kernel(const float* __restrict__ src, half_t* __restrict__ dst, size_t n) {
@@ -523,17 +528,29 @@ void mfma_mlp_forward(hipStream_t stream, const Layout& L, const void* packed, c
     a.packed_halves = (uint32_t)packed_halves(L.net);
     const size_t smem = mfma_fused_smem_bytes(L.net);
     const uint32_t n_tiles = div_round_up(N, 16);
-    auto launch = [&](auto kern, uint32_t tt) {
-        const int occ = occupancy_blocks((const void*)kern, kBlock, smem);
+    auto launch = [&](auto kern, uint32_t tt, int nt) {
+        const int occ = occupancy_blocks((const void*)kern, nt, smem);
         const uint32_t groups = div_round_up(n_tiles, tt);
-        const uint32_t blocks = std::min<uint32_t>(div_round_up(groups, kBlock / 64), (uint32_t)(cu_count() * occ));
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), smem, stream, a, static_cast<const half_t*>(packed),
+        const uint32_t blocks = std::min<uint32_t>(div_round_up(groups, nt / 64), (uint32_t)(cu_count() * occ));
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(nt), smem, stream, a, static_cast<const half_t*>(packed),
                            static_cast<const half_t*>(feat), out);
     };
     switch (L.net.width) {
-        case 32: launch_fwd<32, 2>(a, launch); break;
-        case 64: launch_fwd<64, 2>(a, launch); break;
-        case 128: launch_fwd<128, 1>(a, launch); break;
+        case 32: launch_fwd<32, 2, kBlock>(a, launch); break;
+        case 64: launch_fwd<64, 2, kBlock>(a, launch); break;
+        case 128:
+            // The weights (110 to 150 KB) leave room for one block per CU, so the
+            // block has to bring the waves: 4 of them, one tile each, took 98 us for
+            // 265621 queries of the 144-input network (158 us with the encoding).
+            // Two tiles a wave halve the LDS reads per MFMA; with 32 inputs, whose
+            // fragments are prefetched, 8 waves fit (300001 queries, with the
+            // encoding: 141 -> 100 us, 106 us with 12), else 12 (158 -> 93 us, 99 us
+            // with 8).  While one tile a wave covers the batch, one round of single
+            // tiles is shorter (30000 queries: 42 -> 29.5 us, 33 us with pairs).
+            if (n_tiles <= 8 * (uint32_t)cu_count()) launch_fwd<128, 1, 512>(a, launch);
+            else if (a.k_padded == 32) launch_fwd<128, 2, 512>(a, launch);
+            else launch_fwd<128, 2, 768>(a, launch);
+            break;
         default: fail(NLOD_ERR_UNSUPPORTED, "FP16 MFMA kernels support widths 32, 64 and 128");
     }
     NLOD_LAUNCH_CHECK();
