@@ -582,7 +582,7 @@ __global__ __launch_bounds__(kStageThreads) void bounce_compact_kernel(TracerArg
 
 // ------------------------------------------------------ persistent schedule
 constexpr int kTraceBlock = 768;
-constexpr int kTraceWaves = kTraceBlock / 64;
+constexpr int kTraceBlockSmall = 512;  // 128-wide networks, frames that this many threads per CU hold at once
 constexpr int kSlots = 64;     // rays in flight per wave: one per lane
 constexpr int kInStride = 10;  // floats of one slot's network inputs in LDS (<= 10 used)
 constexpr int kOutStride = 3;  // floats of one slot's network outputs in LDS (<= 3 used)
@@ -597,27 +597,32 @@ __device__ __forceinline__ uint32_t lane_rank(uint64_t mask) {
 // LB: the level's occupancy words are copied into LDS after the weights and
 // the input rows (levels up to about 80^3), so the march's dependent bit
 // reads cost an LDS round trip instead of an L2 one.
-template <int W, int F, int MAXD, bool LB>
-__global__ __launch_bounds__(kTraceBlock, 3) void trace_persistent_kernel(TracerArgs a, NetArgs vis, NetArgs thr,
-                                                                       const half_t* __restrict__ packed_vis,
-                                                                       const half_t* __restrict__ packed_thr,
-                                                                       uint32_t* __restrict__ queue,
-                                                                       float* __restrict__ illum,
-                                                                       uint32_t* __restrict__ inferences,
-                                                                       uint32_t* __restrict__ bounces) {
+// W = 128: LDS holds the visibility weights (110 KB for 32 inputs), which every
+// voxel of a path needs; the throughput network, at most once a bounce, reads
+// its weights from the caches.  480 x 270 paths, 64^3 level, up to 3 bounces:
+// 11.3 ms in the reference schedule (two hundred rounds of a few rays, each nine
+// launches and a host readback), 2.7 ms in this one launch.  12 waves per CU
+// suit large frames (1024 x 1024: 7.6 ms, 8.7 ms with 8), 8 waves those whose
+// rays they hold at once (2.74 against 2.86 ms), which wait for single rays.
+template <int W, int F, int MAXD, bool LB, int BLOCK>
+__global__ __launch_bounds__(BLOCK, BLOCK / 256) void trace_persistent_kernel(
+    TracerArgs a, NetArgs vis, NetArgs thr, const half_t* __restrict__ packed_vis,
+    const half_t* __restrict__ packed_thr, uint32_t* __restrict__ queue, float* __restrict__ illum,
+    uint32_t* __restrict__ inferences, uint32_t* __restrict__ bounces) {
+    constexpr int WAVES = BLOCK / 64;
+    constexpr bool THR_LDS = W < 128;
     extern __shared__ float4 smem4[];
     half_t* sw = reinterpret_cast<half_t*>(smem4);
-    float* s_in = reinterpret_cast<float*>(sw + vis.packed_halves + thr.packed_halves);
-    float* s_out = s_in + kTraceWaves * kSlots * kInStride;
-    for (uint32_t k = threadIdx.x; k < vis.packed_halves / 8; k += kTraceBlock)
-        reinterpret_cast<float4*>(sw + vis.lds_offset)[k] = reinterpret_cast<const float4*>(packed_vis)[k];
-    for (uint32_t k = threadIdx.x; k < thr.packed_halves / 8; k += kTraceBlock)
-        reinterpret_cast<float4*>(sw + thr.lds_offset)[k] = reinterpret_cast<const float4*>(packed_thr)[k];
+    float* s_in = reinterpret_cast<float*>(sw + vis.packed_halves + (THR_LDS ? thr.packed_halves : 0));
+    float* s_out = s_in + WAVES * kSlots * kInStride;
+    stage_weights<BLOCK>(sw + vis.lds_offset, packed_vis, vis.packed_halves);
+    if constexpr (THR_LDS) stage_weights<BLOCK>(sw + thr.lds_offset, packed_thr, thr.packed_halves);
+    const half_t* w_thr = THR_LDS ? sw : packed_thr;
     const uint32_t* bits = a.bits;
     if constexpr (LB) {
-        uint32_t* s_bits = reinterpret_cast<uint32_t*>(s_out + kTraceWaves * kSlots * kOutStride);
+        uint32_t* s_bits = reinterpret_cast<uint32_t*>(s_out + WAVES * kSlots * kOutStride);
         const uint32_t words = (a.R * a.R * a.R + 31u) / 32u;
-        for (uint32_t k = threadIdx.x; k < words; k += kTraceBlock) s_bits[k] = a.bits[k];
+        for (uint32_t k = threadIdx.x; k < words; k += BLOCK) s_bits[k] = a.bits[k];
         bits = s_bits;
     }
     __syncthreads();  // the last block-wide barrier: from here on waves run independently
@@ -706,7 +711,7 @@ __global__ __launch_bounds__(kTraceBlock, 3) void trace_persistent_kernel(Tracer
             const uint32_t q = 16 * t + (uint32_t)n;
             const float* x = rows + (q < cnt ? q : 0u) * kInStride;
             if (use_thr) {
-                const floatx4 o = run_net<W, F, MAXD>(thr, sw, x);
+                const floatx4 o = run_net<W, F, MAXD>(thr, w_thr, x);
                 if (g == 0 && q < cnt) {
 #pragma unroll
                     for (int c = 0; c < 3; ++c) outs[q * kOutStride + c] = act_fwd(thr.out_act, o[c]);
@@ -780,9 +785,10 @@ struct Tracer {
     Model& vis;
     Model& thr;
     bool persistent_ok = false;
+    bool wide_ok = false;  // 128-wide FP16 networks: the persistent launch, with the throughput weights in the caches
     uint32_t F = 2, maxdeg = 4;
-    size_t smem = 0;
-    DevBuf rays_a, rays_b, rays_hit, vis_in, vis_out, thr_in, thr_out, counters, queue;
+    size_t smem = 0;  // weights of the persistent launch
+    DevBuf rays_a, rays_b, rays_hit, vis_in, vis_out, thr_in, thr_out, counters, queue, wide_queue;
     hipEvent_t ev = nullptr;
     uint32_t* host_counts = nullptr;  // pinned readback of the reference schedule's counters
 
@@ -795,15 +801,17 @@ struct Tracer {
             fail(NLOD_ERR_INVALID_ARGUMENT,
                  "the throughput network must take 9 inputs (voxel, wo, wi) or 10 (with the LoD level)");
         if (t.L.net.n_output < 3) fail(NLOD_ERR_INVALID_ARGUMENT, "the throughput network needs 3 outputs");
-        const size_t in_bytes = (size_t)kTraceWaves * kSlots * (kInStride + kOutStride) * sizeof(float);
-        persistent_ok = fused_pair_ok(v, t, kMaxTraceLds - in_bytes);
+        persistent_ok = fused_pair_ok(v, t, kMaxTraceLds - rows_bytes(kTraceBlock));
+        uint32_t Fv, Ft, dv, dt;
+        layout_features(v.L, Fv, dv);
+        layout_features(t.L, Ft, dt);
+        F = Fv;
+        maxdeg = std::max(dv, dt);
         if (persistent_ok) {
-            uint32_t Fv, Ft, dv, dt;
-            layout_features(v.L, Fv, dv);
-            layout_features(t.L, Ft, dt);
-            F = Fv;
-            maxdeg = std::max(dv, dt);
-            smem = mfma_packed_bytes(v.L.net) + mfma_packed_bytes(t.L.net) + in_bytes;
+            smem = mfma_packed_bytes(v.L.net) + mfma_packed_bytes(t.L.net);
+        } else if (v.precision == PREC_FP16 && v.L.net.width == 128 && t.L.net.width == 128 && Fv == Ft) {
+            smem = mfma_packed_bytes(v.L.net);
+            wide_ok = smem + rows_bytes(kTraceBlock) <= kMaxTraceLds;
         }
         NLOD_HIP(hipHostMalloc((void**)&host_counts, 4 * sizeof(uint32_t), hipHostMallocDefault));
         NLOD_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
@@ -812,6 +820,9 @@ struct Tracer {
         if (host_counts) (void)hipHostFree(host_counts);
         if (ev) (void)hipEventDestroy(ev);
     }
+
+    // network inputs and outputs of a block's ray slots
+    static size_t rows_bytes(int threads) { return (size_t)threads * (kInStride + kOutStride) * sizeof(float); }
 
     TracerArgs args(const nlod_camera& cam, const nlod_tracer_params& p, uint32_t sample_idx,
                     uint32_t sample_offset) const {
@@ -875,33 +886,50 @@ struct Tracer {
         vis.require_params(true);
         thr.require_params(true);
         const TracerArgs a = args(cam, p, sample_idx, sample_offset);
-        if (pick(p) == NLOD_TRACER_PERSISTENT) render_persistent(s, a, illum, inferences, bounces);
+        // AUTO with 128-wide networks gives the reference schedule's frame from one launch
+        if (pick(p) == NLOD_TRACER_PERSISTENT || (wide_ok && p.schedule == NLOD_TRACER_AUTO)) render_persistent(s, a, illum, inferences, bounces);
         else render_reference(s, a, illum, inferences, bounces);
     }
 
     void render_persistent(hipStream_t s, const TracerArgs& a, float* illum, uint32_t* inferences,
                            uint32_t* bounces) {
+        DevBuf& queue = wide_ok ? wide_queue : this->queue;  // stats() reports PERSISTENT frames
         queue.ensure(sizeof(uint32_t) * 64);
         const NetArgs av = net_args_of(vis, 0);
-        const NetArgs at = net_args_of(thr, av.packed_halves);
+        const NetArgs at = net_args_of(thr, wide_ok ? 0 : av.packed_halves);
         hipLaunchKernelGGL(reset_queue_kernel, dim3(1), dim3(64), 0, s, queue.as<uint32_t>());
         NLOD_LAUNCH_CHECK();
-        // the level's occupancy words join the weights in LDS when they fit
         const size_t bits_bytes = sizeof(uint32_t) * (((size_t)a.R * a.R * a.R + 31) / 32);
-        const bool lds_bits = smem + bits_bytes <= kMaxTraceLds;
-        const size_t launch_smem = lds_bits ? smem + bits_bytes : smem;
-        dispatch_wf(vis.L.net.width, F, maxdeg, [&](auto Wc, auto Fc, auto Dc) {
+        auto by_block = [&](auto Wc, auto Fc, auto Dc, auto Bc) {
             constexpr int Wv = decltype(Wc)::value, Fv = decltype(Fc)::value, Dv = decltype(Dc)::value;
-            auto kern = lds_bits ? trace_persistent_kernel<Wv, Fv, Dv, true> : trace_persistent_kernel<Wv, Fv, Dv, false>;
-            const int per_cu = std::max(1, occupancy_blocks((const void*)kern, kTraceBlock, launch_smem));
+            constexpr int block = decltype(Bc)::value;
+            // the level's occupancy words join the weights in LDS when they fit
+            size_t launch_smem = smem + rows_bytes(block);
+            const bool lds_bits = launch_smem + bits_bytes <= kMaxTraceLds;
+            if (lds_bits) launch_smem += bits_bytes;
+            auto kern = lds_bits ? trace_persistent_kernel<Wv, Fv, Dv, true, block>
+                                 : trace_persistent_kernel<Wv, Fv, Dv, false, block>;
+            const int per_cu = std::max(1, occupancy_blocks((const void*)kern, block, launch_smem));
             const uint32_t waves_needed = div_round_up(a.n_rays, 16);
             const uint32_t blocks = std::max<uint32_t>(
-                1, std::min<uint32_t>(div_round_up(waves_needed, kTraceWaves), (uint32_t)(cu_count() * per_cu)));
-            hipLaunchKernelGGL(kern, dim3(blocks), dim3(kTraceBlock), launch_smem, s, a, av, at,
+                1, std::min<uint32_t>(div_round_up(waves_needed, block / 64), (uint32_t)(cu_count() * per_cu)));
+            hipLaunchKernelGGL(kern, dim3(blocks), dim3(block), launch_smem, s, a, av, at,
                                static_cast<const half_t*>(vis.packed_fwd(true)),
                                static_cast<const half_t*>(thr.packed_fwd(true)), queue.as<uint32_t>(), illum,
                                inferences, bounces);
-        });
+        };
+        using Block = std::integral_constant<int, kTraceBlock>;
+        using BlockSmall = std::integral_constant<int, kTraceBlockSmall>;
+        if (wide_ok) {
+            dispatch_wf(32, F, maxdeg, [&](auto, auto Fc, auto Dc) {
+                constexpr std::integral_constant<int, 128> Wc{};
+                if (a.n_rays <= (uint32_t)(cu_count() * kTraceBlockSmall)) by_block(Wc, Fc, Dc, BlockSmall{});
+                else by_block(Wc, Fc, Dc, Block{});
+            });
+        } else {
+            dispatch_wf(vis.L.net.width, F, maxdeg,
+                        [&](auto Wc, auto Fc, auto Dc) { by_block(Wc, Fc, Dc, Block{}); });
+        }
         NLOD_LAUNCH_CHECK();
     }
 

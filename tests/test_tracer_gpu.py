@@ -205,6 +205,25 @@ def test_reference_networks_width_128(scene):
     _assert_same(got, ref, "reference networks")
 
 
+@pytest.mark.parametrize("name,w,h", [("default", 80, 60), ("hg", 33, 1), ("roulette", 80, 60), ("stochastic", 80, 60),
+                                      ("log_learning", 80, 60), ("lod0", 41, 30), ("lod2", 400, 400)])
+def test_wide_networks_one_launch_equals_rounds(scene, name, w, h):
+    """128-wide networks: the one launch that AUTO takes against the reference
+    schedule's rounds, bit for bit; frames below and above the block-size switch
+    (131072 rays), levels whose occupancy words fit in LDS (lod2) and do not."""
+    grid, info = scene
+    (vis, _, _), (thr, _, _) = _models(1, seed=17, vis_cfg=configs.REFERENCE_VISIBILITY,
+                                       thr_cfg=configs.REFERENCE_THROUGHPUT)
+    tr = TR.Tracer(grid, vis, thr)
+    cam = _camera(info, w, h)
+    kw = dict({"lod": 1, "max_depth": 3}, **OPTIONS[name])
+    print(f"case wide frame {name} {w}x{h}", flush=True)
+    got = _render(tr, cam, TR.default_params(**kw), 3)
+    ref = _render(tr, cam, TR.default_params(schedule=TR.REFERENCE, **kw), 3)
+    _assert_same(got, ref, name)
+    assert (got[1] >= 1).any()
+
+
 def test_persistent_graph_replays(scene):
     grid, info = scene
     (vis, _, _), (thr, _, _) = _models(1, seed=5)
