@@ -77,6 +77,7 @@ struct TracerArgs {
     float dilation;  // min(inference_min_extent_dilation, voxel_extent_dilation_outward)
     float max_rr_prob, hg_g;
     uint32_t apply_rr, rr_start_bounce, apply_vis_rr, stochastic, use_hg, log_learning;
+    uint32_t slots;  // persistent schedule: rays in flight per wave, 1 .. kSlots
 };
 
 // One path (NeuralBounceQuery + NeuralBounceResult, wavefront_neural_pt.h:43-62).
@@ -583,7 +584,13 @@ __global__ __launch_bounds__(kStageThreads) void bounce_compact_kernel(TracerArg
 // ------------------------------------------------------ persistent schedule
 constexpr int kTraceBlock = 768;
 constexpr int kTraceBlockSmall = 512;  // 128-wide networks, frames that this many threads per CU hold at once
-constexpr int kSlots = 64;     // rays in flight per wave: one per lane
+constexpr int kSlots = 64;     // rays in flight per wave at most: one per lane
+// A wave with few rays left evaluates up to this many voxels ahead of each: a
+// tile has 16 rows either way, and the frame ends with the longest ray, whose
+// voxels otherwise cost one network evaluation after another.  Bounded by that
+// chain: 480 x 270 paths, 128-wide networks, 2.74 -> 1.70 ms (1.78 with 8 ahead);
+// 400 x 300 at 128^3, 64-wide, 5.23 -> 3.72; 1024 x 1024 at 64^3, 9.0 -> 8.7.
+constexpr uint32_t kMaxAhead = 16;
 constexpr int kInStride = 10;  // floats of one slot's network inputs in LDS (<= 10 used)
 constexpr int kOutStride = 3;  // floats of one slot's network outputs in LDS (<= 3 used)
 constexpr size_t kMaxTraceLds = 160 * 1024;  // LDS of one CU
@@ -603,7 +610,8 @@ __device__ __forceinline__ uint32_t lane_rank(uint64_t mask) {
 // 11.3 ms in the reference schedule (two hundred rounds of a few rays, each nine
 // launches and a host readback), 2.7 ms in this one launch.  12 waves per CU
 // suit large frames (1024 x 1024: 7.6 ms, 8.7 ms with 8), 8 waves those whose
-// rays they hold at once (2.74 against 2.86 ms), which wait for single rays.
+// rays they hold at once (2.74 against 2.86 ms), which wait for single rays
+// (these times without the voxels ahead, kMaxAhead).
 template <int W, int F, int MAXD, bool LB, int BLOCK>
 __global__ __launch_bounds__(BLOCK, BLOCK / 256) void trace_persistent_kernel(
     TracerArgs a, NetArgs vis, NetArgs thr, const half_t* __restrict__ packed_vis,
@@ -637,27 +645,29 @@ __global__ __launch_bounds__(BLOCK, BLOCK / 256) void trace_persistent_kernel(
     uint32_t k = 0, b = 0;        // visibility round and bounce of the lane's ray
     uint32_t next = 0, end = 0;   // rays taken from the queue and not yet started
     bool drained = false;
-    // wave-uniform tallies for the frame's statistics: network evaluations
-    // (16-query tiles) and the queries they served, per network, and rounds
+    const uint64_t slots = a.slots >= (uint32_t)kSlots ? ~0ull : (1ull << a.slots) - 1;  // lanes that take rays
+    // tallies for the frame's statistics: network evaluations (16-query tiles)
+    // and the queries they served, per network, and rounds; wave-uniform, but
+    // for n_vis_q, the lane's own checks
     uint32_t n_vis_tiles = 0, n_vis_q = 0, n_thr_tiles = 0, n_thr_q = 0, n_rounds = 0;
     for (;;) {
         // refill free lanes in order from the wave's block of the queue
-        uint64_t free_lanes = __ballot(!live);
+        uint64_t free_lanes = __ballot(!live) & slots;
         while (free_lanes && !drained) {
             if (next == end) {
                 uint32_t start = 0;
-                if (lane == 0) start = atomicAdd(queue, (uint32_t)kSlots);
+                if (lane == 0) start = atomicAdd(queue, a.slots);
                 start = __shfl(start, 0, 64);
                 if (start >= a.n_rays) {
                     drained = true;
                     break;
                 }
                 next = start;
-                end = min(start + (uint32_t)kSlots, a.n_rays);
+                end = min(start + a.slots, a.n_rays);
             }
             const uint32_t take = min((uint32_t)__popcll(free_lanes), end - next);
             const uint32_t rank = lane_rank(free_lanes);
-            if (!live && rank < take) {
+            if (!live && ((slots >> lane) & 1) && rank < take) {
                 raygen(a, next + rank, r);
                 live = true;
                 want = kWantMarch;
@@ -665,7 +675,7 @@ __global__ __launch_bounds__(BLOCK, BLOCK / 256) void trace_persistent_kernel(
                 b = 0;
             }
             next += take;
-            free_lanes = __ballot(!live);
+            free_lanes = __ballot(!live) & slots;
         }
         if (__ballot(live) == 0) break;  // the queue is empty and every lane is done
         ++n_rounds;
@@ -692,16 +702,30 @@ __global__ __launch_bounds__(BLOCK, BLOCK / 256) void trace_persistent_kernel(
         const bool use_thr = n_thr >= n_vis;
         const bool mine = live && want == (use_thr ? kWantThr : kWantVis);
         const uint64_t chosen = __ballot(mine);
-        const uint32_t cnt = (uint32_t)__popcll(chosen);
-        const uint32_t my_row = lane_rank(chosen);
+        const uint32_t rays = (uint32_t)__popcll(chosen);
+        // rows per ray: the voxel it stopped in, then those its march would reach
+        // next if every visibility stayed below its threshold
+        const uint32_t ahead = use_thr || rays > kMaxAhead / 2 ? 1u : kMaxAhead / rays;
+        const uint32_t cnt = rays * ahead;
+        const uint32_t my_row = lane_rank(chosen) * ahead;
+        uint32_t n_rows = 1;  // of this ray that hold a voxel
         if (mine) {
             float in[10];
             if (use_thr) throughput_inputs(a, r, in);
             else visibility_inputs(a, r, in);
             const uint32_t n_in = use_thr ? thr.n_in : 6u;
+            TRay next_r = r;
+            for (uint32_t i = 0;;) {
 #pragma unroll
-            for (int j = 0; j < 10; ++j)
-                if ((uint32_t)j < n_in) rows[my_row * kInStride + j] = in[j];
+                for (int j = 0; j < 10; ++j)
+                    if ((uint32_t)j < n_in) rows[(my_row + i) * kInStride + j] = in[j];
+                if (++i >= ahead) break;
+                // a row past the last voxel repeats the one before it, unused
+                if (n_rows == i && march(a, bits, next_r) && k + i != a.max_vis - 1) {
+                    visibility_inputs(a, next_r, in);
+                    ++n_rows;
+                }
+            }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -729,10 +753,9 @@ __global__ __launch_bounds__(BLOCK, BLOCK / 256) void trace_persistent_kernel(
             n_thr_q += cnt;
         } else {
             n_vis_tiles += tiles;
-            n_vis_q += cnt;
         }
-        if (!mine) continue;
         if (use_thr) {
+            if (!mine) continue;
             float out[3];
 #pragma unroll
             for (int c = 0; c < 3; ++c) out[c] = outs[my_row * kOutStride + c];
@@ -746,23 +769,34 @@ __global__ __launch_bounds__(BLOCK, BLOCK / 256) void trace_persistent_kernel(
                 live = false;
             }
         } else {
-            check_visibility(a, r, outs[my_row * kOutStride], k);
-            if (r.state == kHit) {
-                if (b == a.max_depth - 1) {  // the last bounce keeps no intersection
+            // row by row, as the march and the checks alternate without rows ahead
+            bool checking = mine;
+            for (uint32_t i = 0; i < ahead && checking; ++i) {
+                ++n_vis_q;
+                check_visibility(a, r, outs[(my_row + i) * kOutStride], k);
+                if (r.state == kHit) {
+                    checking = false;
+                    if (b == a.max_depth - 1) {  // the last bounce keeps no intersection
+                        finish(a, r, b, illum, inferences, bounces, true);
+                        live = false;
+                    } else {
+                        want = kWantThr;
+                    }
+                } else if (r.state == kInactive) {
+                    checking = false;
                     finish(a, r, b, illum, inferences, bounces, true);
                     live = false;
                 } else {
-                    want = kWantThr;
+                    ++k;
+                    // the march to the next row's voxel, which ended there before
+                    if (i + 1 < n_rows) march(a, bits, r);
+                    else checking = false, want = kWantMarch;
                 }
-            } else if (r.state == kInactive) {
-                finish(a, r, b, illum, inferences, bounces, true);
-                live = false;
-            } else {
-                ++k;
-                want = kWantMarch;
             }
         }
     }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) n_vis_q += (uint32_t)__shfl_xor((int)n_vis_q, o, 64);
     if (lane == 0) {
         unsigned long long* st = reinterpret_cast<unsigned long long*>(queue + 16);
         atomicAdd(st + 0, (unsigned long long)n_vis_tiles);
@@ -910,10 +944,15 @@ struct Tracer {
             auto kern = lds_bits ? trace_persistent_kernel<Wv, Fv, Dv, true, block>
                                  : trace_persistent_kernel<Wv, Fv, Dv, false, block>;
             const int per_cu = std::max(1, occupancy_blocks((const void*)kern, block, launch_smem));
-            const uint32_t waves_needed = div_round_up(a.n_rays, 16);
+            // A frame that does not fill the chip's waves spreads over them: fewer
+            // rays per wave, more voxels ahead of each (90 x 100 paths at 64^3: 2.04
+            // ms with 64 rays a wave, which leave most waves none, 0.69 ms spread;
+            // 400 x 300 at 128^3: 3.73 and 3.21 ms).
             const uint32_t blocks = std::max<uint32_t>(
-                1, std::min<uint32_t>(div_round_up(waves_needed, block / 64), (uint32_t)(cu_count() * per_cu)));
-            hipLaunchKernelGGL(kern, dim3(blocks), dim3(block), launch_smem, s, a, av, at,
+                1, std::min<uint32_t>(div_round_up(a.n_rays, block / 64), (uint32_t)(cu_count() * per_cu)));
+            TracerArgs al = a;
+            al.slots = std::min<uint32_t>(kSlots, div_round_up(a.n_rays, blocks * (block / 64)));
+            hipLaunchKernelGGL(kern, dim3(blocks), dim3(block), launch_smem, s, al, av, at,
                                static_cast<const half_t*>(vis.packed_fwd(true)),
                                static_cast<const half_t*>(thr.packed_fwd(true)), queue.as<uint32_t>(), illum,
                                inferences, bounces);
