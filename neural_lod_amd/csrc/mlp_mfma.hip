@@ -145,13 +145,15 @@ __device__ __forceinline__ void encode_nongrid(const EncProgram& P, const float*
 }
 
 template <int F, int MAXD, typename TT>
-__global__ __launch_bounds__(kBlock) void encode_kernel(uint32_t N, uint32_t N16, LevelMap map,
-                                                        const EncProgram* __restrict__ prog,
+__global__ __launch_bounds__(kBlock) void encode_kernel(uint32_t N, LevelMap map, const EncProgram* __restrict__ prog,
                                                         const TT* __restrict__ table, const float* __restrict__ in,
-                                                        half_t* __restrict__ feat, const float* __restrict__ xsoa) {
+                                                        QueryRows rows, half_t* __restrict__ feat,
+                                                        const float* __restrict__ xsoa, uint32_t soa_ld) {
     static_assert(std::is_same<TT, half_t>::value, "the encoding pass gathers from the FP16 table copy");
     const EncProgram& P = *prog;
     const uint32_t kp2 = P.k_padded / 2;
+    N = rows.count(N);
+    const uint32_t N16 = (N + 15) / 16 * 16;
     if (blockIdx.y < map.n) {
         // grid rows: two lanes per query (grid_level_h16_pair); N16 is a multiple
         // of 16, so both lanes of a pair return together
@@ -159,7 +161,6 @@ __global__ __launch_bounds__(kBlock) void encode_kernel(uint32_t N, uint32_t N16
         const uint32_t q = t >> 1, lane_s = t & 1u;
         if (q >= N16) return;
         const bool valid = q < N;
-        const float* x = in + (size_t)(valid ? q : 0) * P.n_input_dims;
         const DevSegment& s = P.segs[map.seg[blockIdx.y]];
         const uint32_t level = map.level[blockIdx.y];
         constexpr int VF = F == 1 ? 1 : F / 2;
@@ -167,10 +168,10 @@ __global__ __launch_bounds__(kBlock) void encode_kernel(uint32_t N, uint32_t N16
         float x0, x1, x2;
         if (xsoa) {
             x0 = xsoa[q];
-            x1 = xsoa[N16 + q];
-            x2 = xsoa[2 * (size_t)N16 + q];
+            x1 = xsoa[soa_ld + q];
+            x2 = xsoa[2 * (size_t)soa_ld + q];
         } else {
-            const float* xs = x + s.in_offset;
+            const float* xs = in + (size_t)rows.row(valid ? q : 0) * P.n_input_dims + s.in_offset;
             x0 = xs[0];
             x1 = xs[1];
             x2 = xs[2];
@@ -192,7 +193,7 @@ __global__ __launch_bounds__(kBlock) void encode_kernel(uint32_t N, uint32_t N16
     const uint32_t q = blockIdx.x * kBlock + threadIdx.x;
     if (q >= N16) return;
     const bool valid = q < N;
-    encode_nongrid<MAXD>(P, in + (size_t)(valid ? q : 0) * P.n_input_dims, q, valid, feat);
+    encode_nongrid<MAXD>(P, in + (size_t)rows.row(valid ? q : 0) * P.n_input_dims, q, valid, feat);
 }
 
 // The levels of `lv` (at most kMaxLdsLevels, tables in LDS): one block copies
@@ -200,15 +201,18 @@ __global__ __launch_bounds__(kBlock) void encode_kernel(uint32_t N, uint32_t N16
 // queries, reading the query's position once for all of them.  The gathers come
 // from LDS instead of the L2, which every other level row keeps busy.
 template <int F>
-__global__ __launch_bounds__(kLdsBlock) void encode_lds_kernel(uint32_t N, uint32_t N16, LdsLevels lv,
+__global__ __launch_bounds__(kLdsBlock) void encode_lds_kernel(uint32_t N, LdsLevels lv,
                                                                const EncProgram* __restrict__ prog,
                                                                const half_t* __restrict__ table,
-                                                               const float* __restrict__ in,
+                                                               const float* __restrict__ in, QueryRows rows,
                                                                half_t* __restrict__ feat, float* __restrict__ xsoa,
-                                                               uint32_t soa_off) {
+                                                               uint32_t soa_off, uint32_t soa_ld) {
     extern __shared__ uint4 lds_tab4[];
     half_t* lt = reinterpret_cast<half_t*>(lds_tab4);
     const EncProgram& P = *prog;
+    N = rows.count(N);
+    const uint32_t N16 = (N + 15) / 16 * 16;
+    if (blockIdx.x * kLdsBlock >= N16) return;
     for (uint32_t l = 0; l < lv.n; ++l) {
         const DevSegment& s = P.segs[lv.seg[l]];
         const GridLevels& g = s.lv;
@@ -226,11 +230,11 @@ __global__ __launch_bounds__(kLdsBlock) void encode_lds_kernel(uint32_t N, uint3
     const uint32_t kp2 = P.k_padded / 2;
     for (uint32_t q = blockIdx.x * kLdsBlock + threadIdx.x; q < N16; q += gridDim.x * kLdsBlock) {
         const bool valid = q < N;
-        const float* x = in + (size_t)(valid ? q : 0) * P.n_input_dims;
+        const float* x = in + (size_t)rows.row(valid ? q : 0) * P.n_input_dims;
         if (xsoa) {
             xsoa[q] = x[soa_off];
-            xsoa[N16 + q] = x[soa_off + 1];
-            xsoa[2 * (size_t)N16 + q] = x[soa_off + 2];
+            xsoa[soa_ld + q] = x[soa_off + 1];
+            xsoa[2 * (size_t)soa_ld + q] = x[soa_off + 2];
         }
         for (uint32_t l = 0; l < lv.n; ++l) {
             const DevSegment& s = P.segs[lv.seg[l]];
@@ -268,10 +272,12 @@ struct MlpArgs16 {
 // NT: threads per block (see mfma_mlp_forward).
 template <int W, int TT, int ACT, int KC0, int NT>
 __global__ __launch_bounds__(NT) void mlp_fwd_kernel(MlpArgs16 a, const half_t* __restrict__ packed,
-                                                         const half_t* __restrict__ feat, float* __restrict__ out) {
+                                                     const half_t* __restrict__ feat, QueryRows rows,
+                                                     float* __restrict__ out) {
     constexpr int MT = W / 16, KC = W / 32;
     constexpr int PF = KC0 > 0 ? KC0 : 1;
     const int act = ACT >= 0 ? ACT : a.act;
+    a.N = rows.count(a.N);
     extern __shared__ float4 smem4[];
     half_t* sw = reinterpret_cast<half_t*>(smem4);
     stage_weights<NT>(sw, packed, a.packed_halves);
@@ -370,10 +376,11 @@ __global__ __launch_bounds__(NT) void mlp_fwd_kernel(MlpArgs16 a, const half_t* 
             const uint32_t tile = grp * TT + t;
             const uint32_t q = tile * 16 + n;
             if (tile < n_tiles && q < a.N) {
+                const uint32_t row = rows.row(q);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const uint32_t oi = 4 * g + i;
-                    if (oi < a.n_output) out[(size_t)q * a.n_output + oi] = act_fwd(a.out_act, o[t][i]);
+                    if (oi < a.n_output) out[(size_t)row * a.n_output + oi] = act_fwd(a.out_act, o[t][i]);
                 }
             }
         }
@@ -477,7 +484,7 @@ size_t mfma_pos_scratch_bytes(const Layout& L, uint32_t N) {
 }
 
 void mfma_encode(hipStream_t stream, const Layout& L, const void* d_program, const void* table16, const float* in,
-                 uint32_t N, void* feat, void* pos_scratch) {
+                 uint32_t N, void* feat, void* pos_scratch, QueryRows rows) {
     if (N == 0) return;
     LevelMap map;
     LdsLevels lds;
@@ -499,24 +506,24 @@ void mfma_encode(hipStream_t stream, const Layout& L, const void* d_program, con
             constexpr int F = decltype(Fc)::value;
             NLOD_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(encode_lds_kernel<F>),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsTableBytes));
-            hipLaunchKernelGGL(encode_lds_kernel<F>, dim3(blocks), dim3(kLdsBlock), smem, stream, N, N16, lds,
+            hipLaunchKernelGGL(encode_lds_kernel<F>, dim3(blocks), dim3(kLdsBlock), smem, stream, N, lds,
                                static_cast<const EncProgram*>(d_program), static_cast<const half_t*>(table16), in,
-                               static_cast<half_t*>(feat), xsoa, soa_off);
+                               rows, static_cast<half_t*>(feat), xsoa, soa_off, N16);
         });
         NLOD_LAUNCH_CHECK();
     }
     const dim3 grid(div_round_up(2 * N16, kBlock), map.n + 1);  // grid rows take two lanes per query
     dispatch_fused(L, [&](auto Wc, auto Fc, auto Dc) {
         constexpr int F = decltype(Fc)::value, D = decltype(Dc)::value;
-        hipLaunchKernelGGL((encode_kernel<F, D, half_t>), grid, dim3(kBlock), 0, stream, N, N16, map,
-                           static_cast<const EncProgram*>(d_program), static_cast<const half_t*>(table16), in,
-                           static_cast<half_t*>(feat), (const float*)xsoa);
+        hipLaunchKernelGGL((encode_kernel<F, D, half_t>), grid, dim3(kBlock), 0, stream, N, map,
+                           static_cast<const EncProgram*>(d_program), static_cast<const half_t*>(table16), in, rows,
+                           static_cast<half_t*>(feat), (const float*)xsoa, N16);
     });
     NLOD_LAUNCH_CHECK();
 }
 
 void mfma_mlp_forward(hipStream_t stream, const Layout& L, const void* packed, const void* feat, uint32_t N,
-                      float* out) {
+                      float* out, QueryRows rows) {
     if (N == 0) return;
     MlpArgs16 a{};
     a.N = N;
@@ -533,7 +540,7 @@ void mfma_mlp_forward(hipStream_t stream, const Layout& L, const void* packed, c
         const uint32_t groups = div_round_up(n_tiles, tt);
         const uint32_t blocks = std::min<uint32_t>(div_round_up(groups, nt / 64), (uint32_t)(cu_count() * occ));
         hipLaunchKernelGGL(kern, dim3(blocks), dim3(nt), smem, stream, a, static_cast<const half_t*>(packed),
-                           static_cast<const half_t*>(feat), out);
+                           static_cast<const half_t*>(feat), rows, out);
     };
     switch (L.net.width) {
         case 32: launch_fwd<32, 2, kBlock>(a, launch); break;

@@ -107,6 +107,14 @@ void Model::inference(hipStream_t s, uint32_t N, const float* in, float* out) {
     forward_outputs(s, N, in, out, true);
 }
 
+void Model::inference_rows(hipStream_t s, uint32_t N, QueryRows rows, const float* in, float* out) {
+    require_params(true);
+    if (N == 0) return;
+    ws_feat.ensure(mfma_feature_bytes(L, N));
+    mfma_encode(s, L, program.p, table_half(true), in, N, ws_feat.p, pos_scratch(N), rows);
+    mfma_mlp_forward(s, L, packed_fwd(true), ws_feat.p, N, out, rows);
+}
+
 static size_t enc_bytes(const Layout& L, int precision, uint32_t N) {
     return precision == PREC_FP16 ? mfma_feature_bytes(L, N) : sizeof(float) * (size_t)L.enc_width * N;
 }

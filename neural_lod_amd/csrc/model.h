@@ -19,6 +19,16 @@ enum GradMode : int { GRAD_IGNORE = 0, GRAD_OVERWRITE = 1, GRAD_ACCUMULATE = 2 }
 
 struct Model;
 
+// Which rows of its input and output a batch covers: all (the default), or the
+// first *n entries of `index`, a device list whose length the host does not know
+// (the batch size then only bounds it).
+struct QueryRows {
+    const uint32_t* index = nullptr;
+    const uint32_t* n = nullptr;
+    __device__ __forceinline__ uint32_t count(uint32_t bound) const { return n ? *n : bound; }
+    __device__ __forceinline__ uint32_t row(uint32_t q) const { return index ? index[q] : q; }
+};
+
 // Saved state of one forward pass (tcnn's ForwardContext).
 struct ForwardCtx {
     uint32_t N = 0;
@@ -71,6 +81,8 @@ struct Model {
 
     void encode(hipStream_t s, uint32_t N, const float* in, float* enc_soa, bool inference);
     void inference(hipStream_t s, uint32_t N, const float* in, float* out);
+    // FP16 form, N <= kRecomputeAbove: inference of the listed rows alone
+    void inference_rows(hipStream_t s, uint32_t N, QueryRows rows, const float* in, float* out);
     std::unique_ptr<ForwardCtx> forward(hipStream_t s, uint32_t N, const float* in, float* out, bool use_inference,
                                         bool prepare_input_gradients);
     // forward into an existing context (its buffers only grow)
@@ -132,11 +144,11 @@ size_t mfma_feature_bytes(const Layout& L, uint32_t N);
 // for a [3][N] copy of the grid positions; 0 bytes means the layout does not
 // use one.
 void mfma_encode(hipStream_t stream, const Layout& L, const void* d_program, const void* table16, const float* in,
-                 uint32_t N, void* feat, void* pos_scratch = nullptr);
+                 uint32_t N, void* feat, void* pos_scratch = nullptr, QueryRows rows = {});
 size_t mfma_pos_scratch_bytes(const Layout& L, uint32_t N);
 // MLP on MFMA from the feature fragments -> out float[N][n_output]
 void mfma_mlp_forward(hipStream_t stream, const Layout& L, const void* packed, const void* feat, uint32_t N,
-                      float* out);
+                      float* out, QueryRows rows = {});
 
 
 // ---- mlp_mfma_train.hip (FP16 MFMA training kernels) ------------------------------

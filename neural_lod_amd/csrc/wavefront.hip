@@ -102,6 +102,62 @@ __global__ void gate_kernel(uint32_t N, uint32_t n_vis, uint32_t n_thr, float th
         for (uint32_t i = 0; i < n_thr; ++i) thr_out[(size_t)q * n_thr + i] = 0.0f;
 }
 
+// Split launches of a larger wavefront: the throughput network runs on the
+// segments that reach their threshold only.  Lists them (order does not matter:
+// a query's output does not depend on its batch) and zeroes the other rows.  A
+// block appends its list with one atomic: one per wave, all on one address, cost
+// as much as a network.
+constexpr int kSelectBlock = 1024, kSelectPerThread = 4;
+constexpr uint32_t kSelectQueries = kSelectBlock * kSelectPerThread;
+
+__global__ void zero_count_kernel(uint32_t* count) { *count = 0; }
+
+__global__ __launch_bounds__(kSelectBlock) void select_kernel(uint32_t N, uint32_t n_vis, uint32_t n_thr,
+                                                              float threshold, const float* __restrict__ seg_threshold,
+                                                              const float* __restrict__ vis_out,
+                                                              float* __restrict__ thr_out,
+                                                              uint32_t* __restrict__ index,
+                                                              uint32_t* __restrict__ count) {
+    __shared__ uint32_t s_at[kSelectPerThread * (kSelectBlock / 64)];
+    __shared__ uint32_t s_base;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint64_t mask[kSelectPerThread];
+#pragma unroll
+    for (int r = 0; r < kSelectPerThread; ++r) {
+        const uint32_t q = blockIdx.x * kSelectQueries + r * kSelectBlock + threadIdx.x;
+        bool hit = false;
+        if (q < N) {
+            hit = vis_out[(size_t)q * n_vis] >= (seg_threshold ? seg_threshold[q] : threshold);
+            if (!hit)
+                for (uint32_t i = 0; i < n_thr; ++i) thr_out[(size_t)q * n_thr + i] = 0.0f;
+        }
+        mask[r] = __ballot(hit);
+        if (lane == 0) s_at[r * (kSelectBlock / 64) + wave] = (uint32_t)__popcll(mask[r]);
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {  // exclusive scan of the 64 wave counts
+        const uint32_t v = s_at[lane];
+        uint32_t x = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = (uint32_t)__shfl_up((int)x, o, 64);
+            if (lane >= (uint32_t)o) x += y;
+        }
+        s_at[lane] = x - v;
+        if (lane == 63) s_base = atomicAdd(count, x);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSelectPerThread; ++r) {
+        if (!((mask[r] >> lane) & 1)) continue;
+        const uint32_t below = (uint32_t)__popcll(mask[r] & ((1ull << lane) - 1));
+        index[s_base + s_at[r * (kSelectBlock / 64) + wave] + below] =
+            blockIdx.x * kSelectQueries + r * kSelectBlock + threadIdx.x;
+    }
+}
+static_assert(kSelectPerThread * (kSelectBlock / 64) == 64, "one wave scans the counts");
+constexpr uint32_t kSelectFrom = 16384;  // segments from which the list pays
+
 // wavefront-size buckets of the autotuner: [2^k, 2^(k+2)) for k = 8, 10, ..., 20
 constexpr int kBuckets = 8;
 int bucket_of(uint32_t n) {
@@ -124,6 +180,9 @@ struct Wavefront {
     bool tuned = false;
     int max_blocks_per_cu = 1;
     DevBuf tune_in_v, tune_in_t, tune_out_v, tune_out_t;
+    // visible segments of one pass of the split launches and their number; of
+    // full size from the start, so captured sequences may hold its address
+    DevBuf selected;
     // Captured sequences, keyed by counts and buffers, with the tick of their
     // last use (least recently used goes first beyond kMaxGraphs).  Every graph
     // was captured while both models' epochs had the values in graph_stamp: a
@@ -149,6 +208,7 @@ struct Wavefront {
         fp16 = v.precision == PREC_FP16;
         for (int b = 0; b < kBuckets; ++b) choice[b] = 0;
         if (!fp16) return;
+        selected.ensure(sizeof(uint32_t) * ((size_t)kRecomputeAbove + 1));
         uint32_t Fv, Ft, dv, dt;
         layout_features(v.L, Fv, dv);
         layout_features(t.L, Ft, dt);
@@ -189,6 +249,24 @@ struct Wavefront {
 
     void run_split(hipStream_t s, uint32_t N, const float* vin, const float* tin, float* vout, float* tout,
                    const float* seg_thr = nullptr) {
+        if (fp16 && N >= kSelectFrom) {
+            for (uint32_t q0 = 0; q0 < N; q0 += kRecomputeAbove) {
+                const uint32_t n = std::min(kRecomputeAbove, N - q0);
+                const float* v = vin + (size_t)q0 * vis.L.n_input_dims;
+                float* vo = vout + (size_t)q0 * vis.L.net.n_output;
+                float* to = tout + (size_t)q0 * thr.L.net.n_output;
+                uint32_t* count = selected.as<uint32_t>();
+                vis.inference(s, n, v, vo);
+                hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, s, count);
+                NLOD_LAUNCH_CHECK();
+                hipLaunchKernelGGL(select_kernel, dim3(div_round_up(n, kSelectQueries)), dim3(kSelectBlock), 0, s, n,
+                                   vis.L.net.n_output, thr.L.net.n_output, threshold, seg_thr ? seg_thr + q0 : nullptr,
+                                   vo, to, count + 1, count);
+                NLOD_LAUNCH_CHECK();
+                thr.inference_rows(s, n, QueryRows{count + 1, count}, tin + (size_t)q0 * thr.L.n_input_dims, to);
+            }
+            return;
+        }
         vis.inference(s, N, vin, vout);
         thr.inference(s, N, tin, tout);
         hipLaunchKernelGGL(gate_kernel, dim3(div_round_up(N, 256)), dim3(256), 0, s, N, vis.L.net.n_output,

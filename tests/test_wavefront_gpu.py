@@ -198,3 +198,30 @@ def test_batches_per_segment_thresholds(cuda, precision):
         torch.cuda.synchronize()
         assert torch.equal(vg, ve) and torch.equal(tg, te), f"replay {rep} differs"
         _ = vi.sum().item()
+
+
+@pytest.mark.parametrize("n", [16383, 16384, 16385, 20481, (1 << 20) + 1])
+@pytest.mark.parametrize("share", [0.0, 0.02, 0.5, 1.0])
+def test_split_selects_visible_segments(cuda, n, share):
+    """The split launches list the visible segments and run the throughput
+    network on them alone (from 16384 segments): every row must equal the two
+    networks run in full, gated -- with no segment visible, few, half, all, a
+    list that ends inside a block, and a second pass of one segment."""
+    print(f"case select n={n} share={share}", flush=True)
+    from neural_lod_amd.tcnn import Wavefront
+    _, ((vis, _, _, _), (thr, _, _, _)) = _pair(1)
+    vi, ti = _inputs(n, 3)
+    v, t = vis.inference(vi), thr.inference(ti)
+    lo, hi = float(v.min()), float(v.max())
+    threshold = {0.0: hi + 1.0, 1.0: lo}.get(share)
+    if threshold is None:
+        threshold = float(v[:, 0].float().kthvalue(max(1, int(n * (1 - share)))).values)
+    wf = Wavefront(vis, thr, threshold)
+    out = (torch.full((n, 1), 7.0, device="cuda"), torch.full((n, 3), 7.0, device="cuda"))
+    vo, to = wf.run(vi, ti, shape=0, out=out)
+    assert torch.equal(vo, v)
+    assert torch.equal(to, torch.where(v >= threshold, t, torch.zeros_like(t)))
+    seg = torch.full((n,), threshold, device="cuda")
+    seg[::3] = hi + 1.0
+    vo, to = wf.run(vi, ti, shape=0, out=out, thresholds=seg)
+    assert torch.equal(vo, v) and torch.equal(to, torch.where(v >= seg[:, None], t, torch.zeros_like(t)))
