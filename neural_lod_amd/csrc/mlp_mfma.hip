@@ -1,6 +1,6 @@
 // FP16-MFMA form of the encode + fully fused MLP (gfx950).
 //
-// Three launches per batch:
+// Three launches per batch, two below kLdsFrom queries (without 0.):
 //  0. The coarse levels whose FP16 tables fit in LDS together (72 KB: levels 0
 //     and 1 of the 16^3-based grids): encode_lds_kernel gathers from a copy of
 //     those tables in LDS, sparing the L2 that the other levels saturate.
@@ -410,9 +410,17 @@ __global__ void to_half_kernel(const float* __restrict__ src, half_t* __restrict
         dst[i] = (half_t)src[i];
 }
 
+// Batches from which the LDS pass pays.  It costs a launch whose blocks each copy
+// 70 KB first, 7 us at any size, and spares the level rows 2 of 14 tables: 64-wide
+// networks, 1793 queries 16.9 us with it and 9.8 without, 131072 61.3 and 56.4,
+// 262144 97.7 and 97.3, 524288 199 and 205; 144-input 128-wide one, 265621 queries
+// 93.2 and 89.6.
+constexpr uint32_t kLdsFrom = 300000;
+
 // Splits the grid levels between the LDS pass (levels whose tables still fit,
-// in order) and the rows of the per-level pass (the rest).
-void make_level_maps(const Layout& L, LevelMap& m, LdsLevels& d) {
+// in order) and the rows of the per-level pass (the rest; all levels of a batch
+// of N < kLdsFrom queries).
+void make_level_maps(const Layout& L, uint32_t N, LevelMap& m, LdsLevels& d) {
     m = LevelMap{};
     d = LdsLevels{};
     for (size_t si = 0; si < L.segs.size(); ++si) {
@@ -420,7 +428,7 @@ void make_level_maps(const Layout& L, LevelMap& m, LdsLevels& d) {
         if (s.type != SEG_GRID) continue;
         for (uint32_t l = 0; l < s.n_levels; ++l) {
             const uint32_t halves = (s.levels.offset[l + 1] - s.levels.offset[l]) * s.F;
-            if (d.n < (uint32_t)kMaxLdsLevels && (size_t)(d.halves + halves) * sizeof(half_t) <= kLdsTableBytes) {
+            if (N >= kLdsFrom && d.n < (uint32_t)kMaxLdsLevels && (size_t)(d.halves + halves) * sizeof(half_t) <= kLdsTableBytes) {
                 d.seg[d.n] = (uint8_t)si;
                 d.level[d.n] = (uint8_t)l;
                 d.at[d.n] = d.halves;
@@ -470,7 +478,7 @@ void mfma_to_half(hipStream_t stream, const float* src, void* dst, size_t n) {
 size_t mfma_pos_scratch_bytes(const Layout& L, uint32_t N) {
     LevelMap map;
     LdsLevels lds;
-    make_level_maps(L, map, lds);
+    make_level_maps(L, N, map, lds);
     bool any = false, same = true;
     uint32_t off = 0;
     for (const Segment& s : L.segs) {
@@ -488,7 +496,7 @@ void mfma_encode(hipStream_t stream, const Layout& L, const void* d_program, con
     if (N == 0) return;
     LevelMap map;
     LdsLevels lds;
-    make_level_maps(L, map, lds);
+    make_level_maps(L, N, map, lds);
     const uint32_t N16 = div_round_up(N, 16) * 16;
     // positions as [3][N16], written by the LDS pass and read by the level
     // rows, when every grid segment reads the same 3 inputs
