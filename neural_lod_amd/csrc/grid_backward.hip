@@ -50,6 +50,10 @@ namespace nlod {
 namespace {
 
 constexpr int kBlock = 256;
+// Two blocks of the reduce pass fit in a CU's LDS, so their threads are the
+// waves in flight.  512 against 256 and 1024: training steps of 2^18 queries 536
+// us (547, 552), of 30000 queries 311 us (333, 307).
+constexpr int kReduceBlock = 512;
 constexpr uint32_t kQueriesPerThread = 8;  // count / scatter: loads of 8 queries in flight per thread
 constexpr uint32_t kQueriesPerBlock = kBlock * kQueriesPerThread;
 constexpr uint32_t kTileFloats = 8192;      // values of one tile (kTileFloats / F entries): 64 KiB as int64
@@ -399,13 +403,15 @@ __device__ __forceinline__ unsigned long long to_fixed(float c, int S) {
 
 // Pass 3: group gi of its tile.  The tile's records are its runs in
 // (repetition, query block) order: run j holds run_pre[j + 1] - run_pre[j]
-// records from slot run_addr[j].  Each wave walks a contiguous quarter of the
+// records from slot run_addr[j].  Each wave walks a contiguous eighth of the
 // group, 64 records (one per lane) at a time; a lane keeps the run its record
 // lies in and moves it forward as its record does (a step of 64 records
 // crosses about one run), so the slot of a record costs one or two LDS reads.
+// For small batches, with a few hundred records per tile, what counts are the
+// clearing and writing of the tile and the last, partial batch of each wave.
 // grid: upper bound of groups.
 template <int F>
-__global__ __launch_bounds__(kBlock) void reduce_kernel(uint32_t n_bins, uint32_t n_qblocks,
+__global__ __launch_bounds__(kReduceBlock) void reduce_kernel(uint32_t n_bins, uint32_t n_qblocks,
                                                         const uint32_t* __restrict__ meta,
                                                         const uint32_t* __restrict__ totals,
                                                         const uint32_t* __restrict__ group_start,
@@ -416,8 +422,8 @@ __global__ __launch_bounds__(kBlock) void reduce_kernel(uint32_t n_bins, uint32_
                                                         long long* __restrict__ partial, float* __restrict__ grads,
                                                         int overwrite) {
     constexpr int RW = RecWords<F>::value;
-    constexpr uint32_t kWaves = kBlock / 64;
-    __shared__ unsigned long long acc[kTileFloats];
+    constexpr uint32_t kWaves = kReduceBlock / 64;
+    __shared__ __align__(16) unsigned long long acc[kTileFloats];
     __shared__ uint32_t s_pre[kMaxRuns + 1], s_addr[kMaxRuns];
     const uint32_t gi = blockIdx.x;
     if (gi >= meta[0]) return;
@@ -432,7 +438,7 @@ __global__ __launch_bounds__(kBlock) void reduce_kernel(uint32_t n_bins, uint32_
     const GridBwdBin bin = bins[b];
     const uint32_t n_runs = bin.reps * n_qblocks;  // <= kMaxRuns (pass size)
     const uint32_t total = totals[b];
-    for (uint32_t j = threadIdx.x; j < n_runs; j += kBlock) {
+    for (uint32_t j = threadIdx.x; j < n_runs; j += kReduceBlock) {
         s_pre[j] = run_pre[(size_t)bin.count_row * n_qblocks + j];
         s_addr[j] = run_addr[(size_t)bin.count_row * n_qblocks + j];
     }
@@ -442,10 +448,11 @@ __global__ __launch_bounds__(kBlock) void reduce_kernel(uint32_t n_bins, uint32_
     const uint32_t mbits = meta[3];
     const bool finite = finite_bits(mbits);
     const int S = finite ? fixed_shift(mbits) : 0;
-    for (uint32_t i = threadIdx.x; i < kTileFloats; i += kBlock) acc[i] = 0ull;
+    for (uint32_t i = threadIdx.x; i < kTileFloats / 2; i += kReduceBlock)
+        reinterpret_cast<uint4*>(acc)[i] = uint4{0u, 0u, 0u, 0u};
     __syncthreads();
     // this wave's part of the group: [w0, w1), a multiple of 64 records long
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t per_wave = (end - begin + 64 * kWaves - 1) / (64 * kWaves) * 64;
     const uint32_t w0 = min(end, begin + wave * per_wave), w1 = min(end, w0 + per_wave);
     // the run of record p (p < total): l with s_pre[l] <= p < s_pre[l + 1];
@@ -467,7 +474,7 @@ __global__ __launch_bounds__(kBlock) void reduce_kernel(uint32_t n_bins, uint32_
         return (size_t)s_addr[run] + (p - s_pre[run]);
     };
     // software-pipelined: the next batch's loads are issued before this
-    // batch's LDS adds (lanes past the end load the last record and add 0)
+    // batch's LDS adds (lanes past the end load the last record, unused)
     uint32_t cur[kInFlight][RW] = {}, nxt[kInFlight][RW] = {};  // nxt stays unread after the last batch
     auto load_batch = [&](uint32_t i0, uint32_t (&dst)[kInFlight][RW]) {
         size_t at[kInFlight];
@@ -483,7 +490,9 @@ __global__ __launch_bounds__(kBlock) void reduce_kernel(uint32_t n_bins, uint32_
         if (i1 < w1) load_batch(i1, nxt);
 #pragma unroll
         for (uint32_t k = 0; k < kInFlight; ++k) {
-            const bool valid = i0 + k * 64 + lane < w1;
+            // past the wave's end: lanes that all add to the last record's entries
+            // would take turns at one LDS address
+            if (i0 + k * 64 + lane >= w1) continue;
             const uint32_t key = cur[k][0];
             const bool edge = (key & kEdgeFlag) != 0;
             const uint32_t e0 = key & 0x1fffu, e1 = (key >> 13) & 0x1fffu;
@@ -492,8 +501,8 @@ __global__ __launch_bounds__(kBlock) void reduce_kernel(uint32_t n_bins, uint32_
 #pragma unroll
             for (int f = 0; f < F; ++f) {
                 const float a = __uint_as_float(cur[k][2 + f]);
-                atomicAdd(&acc[e0 * F + f], valid ? fixed(w0f * a) : 0ull);
-                if (edge) atomicAdd(&acc[e1 * F + f], valid ? fixed(wt * a) : 0ull);
+                atomicAdd(&acc[e0 * F + f], fixed(w0f * a));
+                if (edge) atomicAdd(&acc[e1 * F + f], fixed(wt * a));
             }
         }
 #pragma unroll
@@ -505,7 +514,7 @@ __global__ __launch_bounds__(kBlock) void reduce_kernel(uint32_t n_bins, uint32_
     const uint32_t n_vals = bin.n_entries * F;
     if (group_start[b + 1] - group_start[b] == 1) {
         // the tile's only group: this is the gradient
-        for (uint32_t i = threadIdx.x; i < n_vals; i += kBlock) {
+        for (uint32_t i = threadIdx.x; i < n_vals; i += kReduceBlock) {
             const float g = finite ? ldexpf((float)(long long)acc[i], -S) : __uint_as_float(0x7fc00000u);
             float* dst = grads + bin.float_offset + i;
             if (overwrite) *dst = g;
@@ -513,7 +522,7 @@ __global__ __launch_bounds__(kBlock) void reduce_kernel(uint32_t n_bins, uint32_
         }
     } else {
         long long* out = partial + (size_t)gi * kTileFloats;
-        for (uint32_t i = threadIdx.x; i < n_vals; i += kBlock) out[i] = (long long)acc[i];
+        for (uint32_t i = threadIdx.x; i < n_vals; i += kReduceBlock) out[i] = (long long)acc[i];
     }
 }
 
@@ -717,7 +726,7 @@ void GridBackward::run(hipStream_t s, const float* in, uint32_t N, const float* 
         NLOD_LAUNCH_CHECK();
         by_F(F_, [&](auto Fc) {
             constexpr int F = decltype(Fc)::value;
-            hipLaunchKernelGGL(reduce_kernel<F>, dim3((uint32_t)n_groups), dim3(kBlock), 0, s, n_bins_, nqb,
+            hipLaunchKernelGGL(reduce_kernel<F>, dim3((uint32_t)n_groups), dim3(kReduceBlock), 0, s, n_bins_, nqb,
                                meta_.as<uint32_t>(), totals_.as<uint32_t>(), chunk_start_.as<uint32_t>(),
                                d_bins_.as<GridBwdBin>(), counts_.as<uint32_t>(), run_addr_.as<uint32_t>(),
                                records_.as<uint32_t>(), partial_.as<long long>(), grads, ow);
