@@ -30,18 +30,24 @@ struct MlpArgs {
     int32_t act, out_act;
 };
 
-template <int W>
+// Q: queries per lane.  8 (4 at width 128) reuse a staged weight more; batches
+// that give fewer such tiles than there are CUs take 4 (module forward and backward
+// of 20011 queries, 64 x 5: 0.55 -> 0.48 ms; inference of 1000 queries 56 -> 39 us,
+// but of 50000, two small tiles a CU, 98 -> 112 us).
+template <int W, int Q>
 struct Tiling {
-    static constexpr int UB = W / 16;             // units per lane
-    static constexpr int QB = W >= 128 ? 4 : 8;  // queries per lane
-    static constexpr int T = 16 * QB;            // queries per tile
+    static constexpr int UB = W / 16;  // units per lane
+    static constexpr int QB = Q;       // queries per lane
+    static constexpr int T = 16 * QB;  // queries per tile
 };
+template <int W>
+constexpr int kLargeQ = W >= 128 ? 4 : 8;
 
 // acc[UB][QB] += sum_k AT[k][u0 + i] * X[k][q0 + j]; AT is [kk][W] (k-major), X is [kk][T]
-template <int W>
+template <int W, int Q>
 __device__ __forceinline__ void lds_gemm(const float* __restrict__ AT, const float* __restrict__ X, uint32_t kk,
-                                         int u0, int q0, float (&acc)[Tiling<W>::UB][Tiling<W>::QB]) {
-    constexpr int UB = Tiling<W>::UB, QB = Tiling<W>::QB, T = Tiling<W>::T;
+                                         int u0, int q0, float (&acc)[Tiling<W, Q>::UB][Tiling<W, Q>::QB]) {
+    constexpr int UB = Tiling<W, Q>::UB, QB = Tiling<W, Q>::QB, T = Tiling<W, Q>::T;
 #pragma unroll 2
     for (uint32_t k = 0; k < kk; ++k) {
         float a[UB], x[QB];
@@ -96,11 +102,11 @@ __device__ __forceinline__ void load_tile_rows(float* X, const float* __restrict
     }
 }
 
-template <int W>
+template <int W, int Q>
 __global__ __launch_bounds__(kThreads) void mlp_fwd_kernel(uint32_t N, MlpArgs a, const float* __restrict__ w,
                                                            const float* __restrict__ enc, float* __restrict__ out,
                                                            float* __restrict__ hidden) {
-    using Tl = Tiling<W>;
+    using Tl = Tiling<W, Q>;
     constexpr int UB = Tl::UB, QB = Tl::QB, T = Tl::T;
     constexpr int R = W > (int)kChunkK ? W : (int)kChunkK;  // rows of the staging buffers
     extern __shared__ float4 smem4[];
@@ -124,7 +130,7 @@ __global__ __launch_bounds__(kThreads) void mlp_fwd_kernel(uint32_t N, MlpArgs a
             load_tile_rows<T>(bufA, enc, k0, kc, N, tq0);
             stage_transposed(wt, w, W, kc, K, k0, W);
             __syncthreads();
-            lds_gemm<W>(wt, bufA, kc, u0, q0, acc);
+            lds_gemm<W, Q>(wt, bufA, kc, u0, q0, acc);
         }
         float* cur = bufB;
         float* nxt = bufA;
@@ -148,7 +154,7 @@ __global__ __launch_bounds__(kThreads) void mlp_fwd_kernel(uint32_t N, MlpArgs a
             for (int i = 0; i < UB; ++i)
 #pragma unroll
                 for (int j = 0; j < QB; ++j) acc[i][j] = 0.0f;
-            lds_gemm<W>(wt, cur, W, u0, q0, acc);
+            lds_gemm<W, Q>(wt, cur, W, u0, q0, acc);
             float* t = cur;
             cur = nxt;
             nxt = t;
@@ -170,7 +176,7 @@ __global__ __launch_bounds__(kThreads) void mlp_fwd_kernel(uint32_t N, MlpArgs a
 
 // Backward through the layers for a tile: delta_l (SoA [L][W][N], dL/d pre-activation),
 // delta_out (SoA [n_out_padded][N]) and dL/d(enc) (SoA [K][N], optional).
-template <int W>
+template <int W, int Q>
 __global__ __launch_bounds__(kThreads) void mlp_bwd_delta_kernel(uint32_t N, MlpArgs a, const float* __restrict__ w,
                                                                  const float* __restrict__ hidden,
                                                                  const float* __restrict__ out,
@@ -178,7 +184,7 @@ __global__ __launch_bounds__(kThreads) void mlp_bwd_delta_kernel(uint32_t N, Mlp
                                                                  float* __restrict__ delta,
                                                                  float* __restrict__ delta_out,
                                                                  float* __restrict__ d_enc) {
-    using Tl = Tiling<W>;
+    using Tl = Tiling<W, Q>;
     constexpr int UB = Tl::UB, QB = Tl::QB, T = Tl::T;
     constexpr int R = W > (int)kChunkK ? W : (int)kChunkK;
     extern __shared__ float4 smem4[];
@@ -209,7 +215,7 @@ __global__ __launch_bounds__(kThreads) void mlp_bwd_delta_kernel(uint32_t N, Mlp
         for (int i = 0; i < UB; ++i)
 #pragma unroll
             for (int j = 0; j < QB; ++j) acc[i][j] = 0.0f;
-        lds_gemm<W>(wt, bufA, a.n_output, u0, q0, acc);
+        lds_gemm<W, Q>(wt, bufA, a.n_output, u0, q0, acc);
         for (int layer = (int)L - 1; layer >= 0; --layer) {
             // through the hidden activation: delta = acc * act'(h_layer)
 #pragma unroll
@@ -240,7 +246,7 @@ __global__ __launch_bounds__(kThreads) void mlp_bwd_delta_kernel(uint32_t N, Mlp
             for (int i = 0; i < UB; ++i)
 #pragma unroll
                 for (int j = 0; j < QB; ++j) acc[i][j] = 0.0f;
-            lds_gemm<W>(wt, bufB, W, u0, q0, acc);
+            lds_gemm<W, Q>(wt, bufB, W, u0, q0, acc);
         }
         if (!d_enc) continue;
         // dL/d(enc)[m][t] = sum_u W0[u][m] delta_0[u][t], in chunks of W rows of m
@@ -257,7 +263,7 @@ __global__ __launch_bounds__(kThreads) void mlp_bwd_delta_kernel(uint32_t N, Mlp
             for (int i = 0; i < UB; ++i)
 #pragma unroll
                 for (int j = 0; j < QB; ++j) acc[i][j] = 0.0f;
-            lds_gemm<W>(wt, bufB, W, u0, q0, acc);
+            lds_gemm<W, Q>(wt, bufB, W, u0, q0, acc);
 #pragma unroll
             for (int i = 0; i < UB; ++i)
 #pragma unroll
@@ -386,18 +392,28 @@ MlpArgs make_args(const NetShape& n) {
     return MlpArgs{n.n_input, n.n_hidden_layers, n.n_output, n.n_output_padded, n.activation, n.output_activation};
 }
 
-template <int W>
+template <int W, int Q>
 size_t smem_bytes() {
-    constexpr int T = Tiling<W>::T;
+    constexpr int T = Tiling<W, Q>::T;
     constexpr int R = W > (int)kChunkK ? W : (int)kChunkK;
     return sizeof(float) * ((size_t)R * T + (size_t)W * T + (size_t)R * W);
 }
 
-template <int W, typename Kern>
+template <int W, int Q, typename Kern>
 uint32_t grid_for(Kern kern, uint32_t N) {
-    const int occ = occupancy_blocks((const void*)kern, kThreads, smem_bytes<W>());
-    const uint32_t tiles = div_round_up(N, Tiling<W>::T);
+    const int occ = occupancy_blocks((const void*)kern, kThreads, smem_bytes<W, Q>());
+    const uint32_t tiles = div_round_up(N, Tiling<W, Q>::T);
     return std::min<uint32_t>(tiles, (uint32_t)(cu_count() * occ));
+}
+
+// Calls k with the width and the queries per lane that suit N.
+template <typename K>
+void by_tiling(uint32_t W, uint32_t N, K&& k) {
+    by_width(W, [&](auto Wc) {
+        constexpr int Q = kLargeQ<decltype(Wc)::value>;
+        if (Q > 4 && div_round_up(N, 16 * Q) < (uint32_t)cu_count()) k(Wc, std::integral_constant<int, 4>{});
+        else k(Wc, std::integral_constant<int, Q>{});
+    });
 }
 
 uint32_t wgrad_steps(uint32_t N) { return div_round_up(std::max<uint32_t>(N, 1), kWgradQueries); }
@@ -412,11 +428,11 @@ void mlp_forward_f32(hipStream_t stream, const NetShape& net, const float* weigh
                      float* out, float* hidden) {
     if (N == 0) return;
     const MlpArgs a = make_args(net);
-    by_width(net.width, [&](auto Wc) {
-        constexpr int W = decltype(Wc)::value;
-        auto kern = mlp_fwd_kernel<W>;
-        const uint32_t blocks = grid_for<W>(kern, N);
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), smem_bytes<W>(), stream, N, a, weights, enc, out,
+    by_tiling(net.width, N, [&](auto Wc, auto Qc) {
+        constexpr int W = decltype(Wc)::value, Q = decltype(Qc)::value;
+        auto kern = mlp_fwd_kernel<W, Q>;
+        const uint32_t blocks = grid_for<W, Q>(kern, N);
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), (smem_bytes<W, Q>()), stream, N, a, weights, enc, out,
                            hidden);
     });
     NLOD_LAUNCH_CHECK();
@@ -427,11 +443,11 @@ void mlp_backward_delta_f32(hipStream_t stream, const NetShape& net, const float
                             float* d_enc) {
     if (N == 0) return;
     const MlpArgs a = make_args(net);
-    by_width(net.width, [&](auto Wc) {
-        constexpr int W = decltype(Wc)::value;
-        auto kern = mlp_bwd_delta_kernel<W>;
-        const uint32_t blocks = grid_for<W>(kern, N);
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), smem_bytes<W>(), stream, N, a, weights, hidden, out,
+    by_tiling(net.width, N, [&](auto Wc, auto Qc) {
+        constexpr int W = decltype(Wc)::value, Q = decltype(Qc)::value;
+        auto kern = mlp_bwd_delta_kernel<W, Q>;
+        const uint32_t blocks = grid_for<W, Q>(kern, N);
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), (smem_bytes<W, Q>()), stream, N, a, weights, hidden, out,
                            d_out, delta, delta_out, d_enc);
     });
     NLOD_LAUNCH_CHECK();
