@@ -85,8 +85,8 @@ def test_throughput_block_edges(oracle, cuda, n, spp, max_depth):
     tris = S.blob_mesh(20_000, seed=6)
     print(f"case throughput edges n={n} spp={spp} depth={max_depth}", flush=True)
     lb = Labeler(torch.from_numpy(tris).cuda(), 64, 4)
-    longest = [lv["n_list_entries"] / lv["n_occupied"] for lv in lb.levels]
-    assert longest[0] < 8 and longest[-1] > 64  # short and long lists both occur
+    mean = [lv["n_list_entries"] / lv["n_occupied"] for lv in lb.levels]
+    assert mean[0] < 8 and mean[-1] > 32  # of lists of 1 to 427 triangles on the coarsest level
     x, t, v = lb.throughput(n, seed=3, first=10 ** 9, spp=spp, max_depth=max_depth, albedo_seed=8)
     torch.cuda.synchronize()
     ex, et, ev, _ = oracle.throughput_samples(tris, 64, 4, seed=3, first=10 ** 9, n=n, spp=spp, max_depth=max_depth,
