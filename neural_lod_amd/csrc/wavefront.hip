@@ -342,7 +342,7 @@ struct Wavefront {
     // A sequence of wavefronts with host-known sizes, concatenated in the
     // buffers; optionally captured once per size signature and replayed.  A
     // segment's outputs do not depend on its wavefront, so the sequence runs as
-    // one: 20 wavefronts of 3.4M segments one after another, the small ones too
+    // one: 20 wavefronts of 2.7M segments one after another, the small ones too
     // short to fill the chip, took 2.28 ms, together 1.61 ms.
     void run_batches(hipStream_t s, const std::vector<uint32_t>& counts, const float* vin, const float* tin,
                      float* vout, float* tout, bool use_graph, hipStream_t capture_stream,

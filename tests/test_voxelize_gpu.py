@@ -159,6 +159,26 @@ def test_invalid_arguments(cuda):
         V.voxelize(tri, 64, path="fast")
 
 
+@pytest.mark.parametrize("n_tri,at", [(682, 681), (683, 682), (2048, 2047), (349_526, 0), (349_526, 349_525),
+                                      (1_000_000, 700_001)])
+def test_mesh_bbox_block_edges(cuda, n_tri, at):
+    """The box is found in whichever block holds the extreme triangle: around
+    one tile of 6144 floats (682.67 triangles), at three whole tiles, past the
+    tiles of one sweep of two blocks per CU (349,525 triangles on 256 CUs), and
+    with infinities beside the finite coordinates."""
+    from neural_lod_amd import voxelizer as V
+    rng = np.random.default_rng(n_tri)
+    tris = rng.normal(size=(n_tri, 9)).astype(np.float32)
+    tris[at, 1] = -1e4
+    tris[at, 3] = np.inf
+    tris[at, 8] = 1e4
+    print(f"case bbox n_tri={n_tri} at={at}", flush=True)
+    mn, mx = V.mesh_bbox(torch.from_numpy(tris).cuda())
+    v = tris.reshape(-1, 3)
+    np.testing.assert_array_equal(mn, v.min(axis=0))
+    np.testing.assert_array_equal(mx, v.max(axis=0))
+
+
 @pytest.mark.parametrize("n_tri", [1, 2, 3, 4, 5, 7, 1000, 200_001])
 @pytest.mark.parametrize("offset", [0, 1])
 def test_mesh_bbox(cuda, n_tri, offset):
