@@ -42,7 +42,7 @@ COMMON_FLAGS = [
 # so the activation code reads them without v_accvgpr_read copies
 FILE_FLAGS = {
     name: ["-mllvm", "-amdgpu-mfma-vgpr-form"]
-    for name in ("mlp_mfma.hip", "mlp_mfma_train.hip", "mlp_mfma_fused_train.hip", "wavefront.hip")
+    for name in ("mlp_fp32.hip", "mlp_mfma.hip", "mlp_mfma_train.hip", "mlp_mfma_fused_train.hip", "wavefront.hip")
 }
 
 

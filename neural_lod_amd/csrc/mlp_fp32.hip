@@ -1,14 +1,27 @@
 // Plain FP32 form of the fully fused MLP (tiny-cuda-nn src/fully_fused_mlp.cu,
 // no biases): forward, backward through the layers, and weight gradients.
 //
-// A workgroup of 256 lanes owns a tile of T queries and keeps the tile's
-// activations in LDS ([unit][query], FP32).  Each layer is an LDS-resident
-// GEMM out[W][T] = A[W][K] . in[K][T]: the current weight matrix is staged
-// k-major in LDS, and every lane accumulates a (W/16 units x T/16 queries)
-// register block with FP32 FMAs (one float4 of weights and T/64 float4s of
-// activations per 4*(T/16)... FMAs).  Weight gradients are batch reductions
-// dW = delta . act^T on FP32 MFMAs, split over query chunks, with a
-// deterministic second-pass reduction.
+// Every product runs on v_mfma_f32_16x16x4_f32 (FP32 operands, products and
+// sums).  A wave owns 16 queries and keeps their activations in registers
+// from the first layer to the last: the accumulator layout (lane group
+// g = lane / 16 holds units 16t + 4g .. 16t + 4g + 3 of query lane % 16) is, one
+// register at a time, the B operand of four products over the units
+// {16t + 4g' + r, g' = 0..3}.  The matching A operands are four consecutive
+// floats of a weight row, one 16-byte LDS read in the forward pass; the backward
+// pass reads the same staged rows transposed, a dword at a time.  Only the
+// current weight matrix is in LDS, staged by the block as it lies in memory; the
+// next one is loaded into registers while the current one is used.  Weight
+// gradients are batch reductions dW = delta . act^T, split over query chunks,
+// with a deterministic second-pass reduction.
+//
+// Bound: the FP32 matrix rate for large batches; below two tiles a CU the serial
+// chain of one wave (layers x products of 32 cycles, the weight loads between
+// them).  Blocks of FP32 FMAs per lane, with the weights transposed on their way
+// into LDS (all 64 lanes of a store on one bank), took, encoding included: 64 x 4
+// network, 1000 queries 49 us, now 15; 20011, 76 and 38; 2^20, 1382 and 931;
+// 128 x 4 network 89 and 33, 206 and 65, 5252 and 1727.  Two query tiles per wave
+// (each weight staged for twice the queries) gave 899 us for the 931, three waves
+// per SIMD by spilling 968.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -22,255 +35,264 @@
 namespace nlod {
 namespace {
 
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
 constexpr int kThreads = 256;
-constexpr uint32_t kChunkK = 64;  // layer-0 / d_enc rows handled per pass
+constexpr int kChunkK = 64;  // columns of the first matrix staged at a time
+constexpr uint32_t kTile = 16 * (kThreads / 64);  // queries per block: 16 per wave
 
 struct MlpArgs {
     uint32_t n_input, n_hidden_layers, n_output, n_output_padded;
     int32_t act, out_act;
 };
 
-// Q: queries per lane.  8 (4 at width 128) reuse a staged weight more; batches
-// that give fewer such tiles than there are CUs take 4 (module forward and backward
-// of 20011 queries, 64 x 5: 0.55 -> 0.48 ms; inference of 1000 queries 56 -> 39 us,
-// but of 50000, two small tiles a CU, 98 -> 112 us).
-template <int W, int Q>
-struct Tiling {
-    static constexpr int UB = W / 16;  // units per lane
-    static constexpr int QB = Q;       // queries per lane
-    static constexpr int T = 16 * QB;  // queries per tile
-};
+// Floats between the staged rows: 4 mod 16, so that neither the 16-byte reads of
+// 16 rows nor the dword reads of 4 x 16 (rows 4 apart, columns consecutive) meet
+// in an LDS bank.
 template <int W>
-constexpr int kLargeQ = W >= 128 ? 4 : 8;
+constexpr int kLd = (W > kChunkK ? W : kChunkK) + 4;
 
-// acc[UB][QB] += sum_k AT[k][u0 + i] * X[k][q0 + j]; AT is [kk][W] (k-major), X is [kk][T]
-template <int W, int Q>
-__device__ __forceinline__ void lds_gemm(const float* __restrict__ AT, const float* __restrict__ X, uint32_t kk,
-                                         int u0, int q0, float (&acc)[Tiling<W, Q>::UB][Tiling<W, Q>::QB]) {
-    constexpr int UB = Tiling<W, Q>::UB, QB = Tiling<W, Q>::QB, T = Tiling<W, Q>::T;
-#pragma unroll 2
-    for (uint32_t k = 0; k < kk; ++k) {
-        float a[UB], x[QB];
+// R rows x up to C columns (multiples of 4) of a row-major matrix, on their way
+// into LDS: load() into registers, store() behind the barrier that frees the
+// buffer.  Rows start at any multiple of 4 bytes.
+template <int R, int C>
+struct Staged {
+    static constexpr int kLanes = C / 4, kRows = kThreads / kLanes, kSteps = (R + kRows - 1) / kRows;
+    floatx4 v[kSteps];
+    __device__ __forceinline__ void load(const float* __restrict__ src, uint32_t rows, uint32_t cols, uint32_t ld) {
+        const uint32_t c = threadIdx.x % kLanes * 4;
 #pragma unroll
-        for (int i = 0; i < UB; i += (UB >= 4 ? 4 : UB)) {
-            if constexpr (UB >= 4) {
-                const float4 v = *reinterpret_cast<const float4*>(AT + k * W + u0 + i);
-                a[i] = v.x; a[i + 1] = v.y; a[i + 2] = v.z; a[i + 3] = v.w;
-            } else {
-#pragma unroll
-                for (int t = 0; t < UB; ++t) a[t] = AT[k * W + u0 + t];
-            }
+        for (int i = 0; i < kSteps; ++i) {
+            const uint32_t r = threadIdx.x / kLanes + i * kRows;
+            v[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+            if (r < rows && c < cols) __builtin_memcpy(&v[i], src + (size_t)r * ld + c, 16);
         }
+    }
+    __device__ __forceinline__ void store(float* dst, uint32_t ld) const {
+        const uint32_t c = threadIdx.x % kLanes * 4;
 #pragma unroll
-        for (int j = 0; j < QB; j += 4) {
-            const float4 v = *reinterpret_cast<const float4*>(X + k * T + q0 + j);
-            x[j] = v.x; x[j + 1] = v.y; x[j + 2] = v.z; x[j + 3] = v.w;
+        for (int i = 0; i < kSteps; ++i) {
+            const uint32_t r = threadIdx.x / kLanes + i * kRows;
+            if (R % kRows == 0 || r < (uint32_t)R) *reinterpret_cast<floatx4*>(dst + r * ld + c) = v[i];
         }
+    }
+};
+
+__device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// The W = 16 MT sums of a layer for 16 queries.  Input tiles alternate between two
+// accumulators: half the chain of dependent products, and half the rounding
+// errors in a row (against 64 bits, 64 x 5 and 128 x 4 networks: the outputs' relative
+// error 2.0e-7 and 2.8e-7, 2.8e-7 and 3.8e-7 with one accumulator).
+template <int MT>
+struct Sums {
+    floatx4 v[2][MT];
+    __device__ __forceinline__ void clear() {
 #pragma unroll
-        for (int i = 0; i < UB; ++i)
+        for (int m = 0; m < MT; ++m) v[0][m] = v[1][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    __device__ __forceinline__ floatx4 sum(int m) const { return v[0][m] + v[1][m]; }
+
+    // sums[m] += A[16m + .][16k .. 16k + 15] . x: 16 input units, held as an accumulator tile
+    __device__ __forceinline__ void add_rows(const float* __restrict__ A, uint32_t ld, int k, floatx4 x) {
+        const uint32_t lane = threadIdx.x & 63, g = lane >> 4, m16 = lane & 15;
+        floatx4 a[MT];
 #pragma unroll
-            for (int j = 0; j < QB; ++j) acc[i][j] += a[i] * x[j];
+        for (int m = 0; m < MT; ++m)
+            a[m] = *reinterpret_cast<const floatx4*>(A + (16 * m + m16) * ld + 16 * k + 4 * g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) v[k & 1][m] = mfma4(a[m][r], x[r], v[k & 1][m]);
     }
-}
-
-// Stage rows [r0, r0+rows) x cols of a row-major matrix (stride ld) into LDS,
-// transposed to [col][W-strided row]: dst[c * W + (r - r0)].
-__device__ __forceinline__ void stage_transposed(float* dst, const float* __restrict__ src, uint32_t rows,
-                                                 uint32_t cols, uint32_t ld, uint32_t col0, uint32_t Wd) {
-    for (uint32_t idx = threadIdx.x; idx < rows * cols; idx += kThreads) {
-        const uint32_t r = idx / cols, c = idx - r * cols;
-        dst[c * Wd + r] = src[(size_t)r * ld + col0 + c];
+    // sums[m] += A[16k .. 16k + 15][16m + .]^T . x
+    __device__ __forceinline__ void add_cols(const float* __restrict__ A, uint32_t ld, int k, floatx4 x) {
+        const uint32_t lane = threadIdx.x & 63, g = lane >> 4, m16 = lane & 15;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float a[MT];
+#pragma unroll
+            for (int m = 0; m < MT; ++m) a[m] = A[(16 * k + 4 * g + r) * ld + 16 * m + m16];
+#pragma unroll
+            for (int m = 0; m < MT; ++m) v[k & 1][m] = mfma4(a[m], x[r], v[k & 1][m]);
+        }
     }
-}
+};
 
-// Stage rows [k0, k0+kk) of a row-major [*, ld] matrix as-is: dst[k * ld + m].
-__device__ __forceinline__ void stage_rows(float* dst, const float* __restrict__ src, uint32_t kk, uint32_t ld,
-                                           uint32_t m0, uint32_t mm, uint32_t Wd) {
-    for (uint32_t idx = threadIdx.x; idx < kk * mm; idx += kThreads) {
-        const uint32_t k = idx / mm, m = idx - k * mm;
-        dst[k * Wd + m] = src[(size_t)k * ld + m0 + m];
-    }
-}
-
-// Load rows [k0, k0+kk) of a SoA [*][N] global matrix for the tile into X[kk][T] (0 beyond N).
-template <int T>
-__device__ __forceinline__ void load_tile_rows(float* X, const float* __restrict__ src, uint32_t k0, uint32_t kk,
-                                               uint32_t N, uint32_t tq0) {
-    for (uint32_t idx = threadIdx.x; idx < kk * T; idx += kThreads) {
-        const uint32_t k = idx / T, q = idx - k * T;
-        X[idx] = (tq0 + q < N) ? src[(size_t)(k0 + k) * N + tq0 + q] : 0.0f;
-    }
-}
-
-template <int W, int Q>
-__global__ __launch_bounds__(kThreads) void mlp_fwd_kernel(uint32_t N, MlpArgs a, const float* __restrict__ w,
-                                                           const float* __restrict__ enc, float* __restrict__ out,
-                                                           float* __restrict__ hidden) {
-    using Tl = Tiling<W, Q>;
-    constexpr int UB = Tl::UB, QB = Tl::QB, T = Tl::T;
-    constexpr int R = W > (int)kChunkK ? W : (int)kChunkK;  // rows of the staging buffers
+template <int W>
+__global__ __launch_bounds__(kThreads, W >= 128 ? 1 : 2) void mlp_fwd_kernel(uint32_t N, MlpArgs a, const float* __restrict__ w,
+                                               const float* __restrict__ enc, float* __restrict__ out,
+                                               float* __restrict__ hidden) {
+    constexpr int MT = W / 16, LD = kLd<W>;
     extern __shared__ float4 smem4[];
-    float* bufA = reinterpret_cast<float*>(smem4);  // [R][T]
-    float* bufB = bufA + R * T;                      // [W][T]
-    float* wt = bufB + W * T;                        // [R][W]
-    const int tu = threadIdx.x >> 4, tq = threadIdx.x & 15;
-    const int u0 = tu * UB, q0 = tq * QB;
-    const uint32_t K = a.n_input;
-    const uint32_t n_tiles = (N + T - 1) / T;
+    float* w_lds = reinterpret_cast<float*>(smem4);  // [W][LD]: the current matrix
+    float* out_lds = w_lds + W * LD;                 // [16][LD]: the output matrix
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, n16 = lane & 15;
+    const uint32_t K = a.n_input, L = a.n_hidden_layers;
+    const float* w_hidden = w + (size_t)W * K;  // L - 1 matrices [W][W]
+    {
+        Staged<16, W> so;
+        so.load(w_hidden + (size_t)(L - 1) * W * W, a.n_output, W, W);
+        so.store(out_lds, LD);
+    }
+    const uint32_t n_tiles = (N + kTile - 1) / kTile;
     for (uint32_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        const uint32_t tq0 = tile * T;
-        float acc[UB][QB];
-#pragma unroll
-        for (int i = 0; i < UB; ++i)
-#pragma unroll
-            for (int j = 0; j < QB; ++j) acc[i][j] = 0.0f;
+        const uint32_t q = tile * kTile + wave * 16 + n16;
+        const bool valid = q < N;
+        Sums<MT> acc;
+        acc.clear();
+        Staged<W, kChunkK> s0;
+        s0.load(w, W, min((uint32_t)kChunkK, K), K);
         for (uint32_t k0 = 0; k0 < K; k0 += kChunkK) {
-            const uint32_t kc = min(kChunkK, K - k0);
-            __syncthreads();
-            load_tile_rows<T>(bufA, enc, k0, kc, N, tq0);
-            stage_transposed(wt, w, W, kc, K, k0, W);
-            __syncthreads();
-            lds_gemm<W, Q>(wt, bufA, kc, u0, q0, acc);
-        }
-        float* cur = bufB;
-        float* nxt = bufA;
-        for (uint32_t layer = 0;; ++layer) {
-            // activation -> LDS tile (and the saved activations for backward)
+            const uint32_t kc = min((uint32_t)kChunkK, K - k0);  // a multiple of 16
+            floatx4 x[kChunkK / 16];
 #pragma unroll
-            for (int i = 0; i < UB; ++i) act_fwd_n<QB>(a.act, acc[i]);
+            for (int c = 0; c < kChunkK / 16; ++c)
 #pragma unroll
-            for (int i = 0; i < UB; ++i)
-#pragma unroll
-                for (int j = 0; j < QB; ++j) {
-                    const float h = acc[i][j];
-                    cur[(u0 + i) * T + q0 + j] = h;
-                    if (hidden && tq0 + q0 + j < N) hidden[((size_t)layer * W + u0 + i) * N + tq0 + q0 + j] = h;
+                for (int r = 0; r < 4; ++r) {
+                    const uint32_t k = 16 * c + 4 * g + r;
+                    x[c][r] = k < kc && valid ? enc[(size_t)(k0 + k) * N + q] : 0.0f;
                 }
-            if (layer + 1 >= a.n_hidden_layers) break;
             __syncthreads();
-            stage_transposed(wt, w + (size_t)W * K + (size_t)layer * W * W, W, W, W, 0, W);
+            s0.store(w_lds, LD);
             __syncthreads();
+            if (k0 + kChunkK < K) s0.load(w + k0 + kChunkK, W, min((uint32_t)kChunkK, K - k0 - kChunkK), K);
 #pragma unroll
-            for (int i = 0; i < UB; ++i)
-#pragma unroll
-                for (int j = 0; j < QB; ++j) acc[i][j] = 0.0f;
-            lds_gemm<W, Q>(wt, cur, W, u0, q0, acc);
-            float* t = cur;
-            cur = nxt;
-            nxt = t;
+            for (int c = 0; c < kChunkK / 16; ++c)
+                if (16u * c < kc) acc.add_rows(w_lds, LD, c, x[c]);
         }
-        __syncthreads();
-        // output layer: lane t < T computes query t's outputs (weights broadcast from global/L1)
-        const float* w_out = w + (size_t)W * K + (size_t)(a.n_hidden_layers - 1) * W * W;
-        for (uint32_t t = threadIdx.x; t < (uint32_t)T; t += kThreads) {
-            if (tq0 + t >= N) continue;
-            for (uint32_t r = 0; r < a.n_output; ++r) {
-                float s = 0.0f;
-#pragma unroll 8
-                for (int k = 0; k < W; ++k) s += w_out[r * W + k] * cur[k * T + t];
-                out[(size_t)(tq0 + t) * a.n_output + r] = act_fwd(a.out_act, s);
+        Staged<W, W> s;
+        if (L > 1) s.load(w_hidden, W, W, W);
+        floatx4 h[MT];
+        for (uint32_t layer = 0;; ++layer) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const floatx4 z = acc.sum(m);
+                float y[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) y[r] = z[r];
+                act_fwd_n<4>(a.act, y);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    h[m][r] = y[r];
+                    if (hidden && valid) hidden[((size_t)layer * W + 16 * m + 4 * g + r) * N + q] = y[r];
+                }
             }
+            if (layer + 1 >= L) break;
+            __syncthreads();
+            s.store(w_lds, LD);
+            __syncthreads();
+            if (layer + 2 < L) s.load(w_hidden + (size_t)(layer + 1) * W * W, W, W, W);
+            acc.clear();
+#pragma unroll
+            for (int k = 0; k < MT; ++k) acc.add_rows(w_lds, LD, k, h[k]);
         }
+        Sums<1> o;
+        o.clear();
+#pragma unroll
+        for (int k = 0; k < MT; ++k) o.add_rows(out_lds, LD, k, h[k]);
+        const floatx4 z = o.sum(0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (4 * g + r < a.n_output && valid) out[(size_t)q * a.n_output + 4 * g + r] = act_fwd(a.out_act, z[r]);
     }
 }
 
 // Backward through the layers for a tile: delta_l (SoA [L][W][N], dL/d pre-activation),
 // delta_out (SoA [n_out_padded][N]) and dL/d(enc) (SoA [K][N], optional).
-template <int W, int Q>
-__global__ __launch_bounds__(kThreads) void mlp_bwd_delta_kernel(uint32_t N, MlpArgs a, const float* __restrict__ w,
-                                                                 const float* __restrict__ hidden,
-                                                                 const float* __restrict__ out,
-                                                                 const float* __restrict__ d_out,
-                                                                 float* __restrict__ delta,
-                                                                 float* __restrict__ delta_out,
-                                                                 float* __restrict__ d_enc) {
-    using Tl = Tiling<W, Q>;
-    constexpr int UB = Tl::UB, QB = Tl::QB, T = Tl::T;
-    constexpr int R = W > (int)kChunkK ? W : (int)kChunkK;
+template <int W>
+__global__ __launch_bounds__(kThreads, W >= 128 ? 1 : 2) void mlp_bwd_delta_kernel(uint32_t N, MlpArgs a, const float* __restrict__ w,
+                                                     const float* __restrict__ hidden, const float* __restrict__ out,
+                                                     const float* __restrict__ d_out, float* __restrict__ delta,
+                                                     float* __restrict__ delta_out, float* __restrict__ d_enc) {
+    constexpr int MT = W / 16, LD = kLd<W>;
     extern __shared__ float4 smem4[];
-    float* bufA = reinterpret_cast<float*>(smem4);  // [R][T]
-    float* bufB = bufA + R * T;                      // [W][T]
-    float* wt = bufB + W * T;                        // [R][W]
-    const int tu = threadIdx.x >> 4, tq = threadIdx.x & 15;
-    const int u0 = tu * UB, q0 = tq * QB;
+    float* w_lds = reinterpret_cast<float*>(smem4);  // [W][LD]: the current matrix
+    float* out_lds = w_lds + W * LD;                 // [16][LD]: the output matrix
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, n16 = lane & 15;
     const uint32_t K = a.n_input, L = a.n_hidden_layers;
-    const uint32_t n_tiles = (N + T - 1) / T;
+    const float* w_hidden = w + (size_t)W * K;
+    {
+        Staged<16, W> so;
+        so.load(w_hidden + (size_t)(L - 1) * W * W, a.n_output, W, W);
+        so.store(out_lds, LD);
+    }
+    __syncthreads();
+    const uint32_t n_tiles = (N + kTile - 1) / kTile;
     for (uint32_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        const uint32_t tq0 = tile * T;
-        __syncthreads();
-        // output activation transfer (fully_fused_mlp.cu:757-760): dz[r][t] in bufA rows 0..15
-        for (uint32_t idx = threadIdx.x; idx < 16u * T; idx += kThreads) {
-            const uint32_t r = idx / T, t = idx - r * T, q = tq0 + t;
-            float v = 0.0f;
-            if (q < N && r < a.n_output)
-                v = d_out[(size_t)q * a.n_output + r] * act_bwd(a.out_act, out[(size_t)q * a.n_output + r]);
-            bufA[idx] = v;
-            if (q < N && r < a.n_output_padded) delta_out[(size_t)r * N + q] = v;
+        const uint32_t q = tile * kTile + wave * 16 + n16;
+        const bool valid = q < N;
+        floatx4 hv[MT];  // the layer's activations
+        auto load_hidden = [&](uint32_t layer) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    hv[m][r] = valid ? hidden[((size_t)layer * W + 16 * m + 4 * g + r) * N + q] : 0.0f;
+        };
+        // output activation transfer (fully_fused_mlp.cu:757-760)
+        floatx4 dz;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t row = 4 * g + r;
+            dz[r] = 0.0f;
+            if (valid && row < a.n_output)
+                dz[r] = d_out[(size_t)q * a.n_output + row] * act_bwd(a.out_act, out[(size_t)q * a.n_output + row]);
+            if (valid && row < a.n_output_padded) delta_out[(size_t)row * N + q] = dz[r];
         }
-        // W_out [16][W] row-major is already k-major for the transposed product
-        stage_rows(wt, w + (size_t)W * K + (size_t)(L - 1) * W * W, a.n_output, W, 0, W, W);
-        __syncthreads();
-        float acc[UB][QB];
-#pragma unroll
-        for (int i = 0; i < UB; ++i)
-#pragma unroll
-            for (int j = 0; j < QB; ++j) acc[i][j] = 0.0f;
-        lds_gemm<W, Q>(wt, bufA, a.n_output, u0, q0, acc);
-        for (int layer = (int)L - 1; layer >= 0; --layer) {
+        load_hidden(L - 1);
+        Staged<W, W> s;
+        if (L > 1) s.load(w_hidden + (size_t)(L - 2) * W * W, W, W, W);
+        Sums<MT> acc;
+        acc.clear();
+        acc.add_cols(out_lds, LD, 0, dz);
+        floatx4 d[MT];
+        for (uint32_t layer = L; layer-- > 0;) {
             // through the hidden activation: delta = acc * act'(h_layer)
 #pragma unroll
-            for (int i = 0; i < UB; ++i) {
-                float hv[QB], dv[QB];
+            for (int m = 0; m < MT; ++m) {
+                const floatx4 z = acc.sum(m);
+                float y[4], dv[4];
 #pragma unroll
-                for (int j = 0; j < QB; ++j) {
-                    const uint32_t q = tq0 + q0 + j;
-                    hv[j] = q < N ? hidden[((size_t)layer * W + u0 + i) * N + q] : 0.0f;
-                }
-                act_bwd_n<QB>(a.act, hv, dv);
+                for (int r = 0; r < 4; ++r) y[r] = hv[m][r];
+                act_bwd_n<4>(a.act, y, dv);
 #pragma unroll
-                for (int j = 0; j < QB; ++j) {
-                    const uint32_t q = tq0 + q0 + j;
-                    acc[i][j] *= dv[j];
-                    if (q < N) delta[((size_t)layer * W + u0 + i) * N + q] = acc[i][j];
+                for (int r = 0; r < 4; ++r) {
+                    d[m][r] = z[r] * dv[r];
+                    if (valid) delta[((size_t)layer * W + 16 * m + 4 * g + r) * N + q] = d[m][r];
                 }
             }
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < UB; ++i)
-#pragma unroll
-                for (int j = 0; j < QB; ++j) bufB[(u0 + i) * T + q0 + j] = acc[i][j];
             if (layer == 0) break;
-            stage_rows(wt, w + (size_t)W * K + (size_t)(layer - 1) * W * W, W, W, 0, W, W);
             __syncthreads();
+            s.store(w_lds, LD);
+            __syncthreads();
+            load_hidden(layer - 1);
+            if (layer > 1) s.load(w_hidden + (size_t)(layer - 2) * W * W, W, W, W);
+            acc.clear();
 #pragma unroll
-            for (int i = 0; i < UB; ++i)
-#pragma unroll
-                for (int j = 0; j < QB; ++j) acc[i][j] = 0.0f;
-            lds_gemm<W, Q>(wt, bufB, W, u0, q0, acc);
+            for (int k = 0; k < MT; ++k) acc.add_cols(w_lds, LD, k, d[k]);
         }
         if (!d_enc) continue;
-        // dL/d(enc)[m][t] = sum_u W0[u][m] delta_0[u][t], in chunks of W rows of m
-        for (uint32_t m0 = 0; m0 < K; m0 += W) {
-            const uint32_t mm = min((uint32_t)W, K - m0);
+        // dL/d(enc)[m][q] = sum_u W0[u][m] delta_0[u][q]
+        for (uint32_t m0 = 0; m0 < K; m0 += kChunkK) {
+            const uint32_t mc = min((uint32_t)kChunkK, K - m0);
+            Staged<W, kChunkK> s0;
+            s0.load(w + m0, W, mc, K);
             __syncthreads();
-            stage_rows(wt, w, W, K, m0, mm, W);
-            for (uint32_t idx = threadIdx.x; idx < (uint32_t)W * (W - mm); idx += kThreads) {
-                const uint32_t k = idx / (W - mm), m = mm + idx % (W - mm);
-                wt[k * W + m] = 0.0f;
+            s0.store(w_lds, LD);
+            __syncthreads();
+            for (uint32_t m = 0; m < mc; m += 16) {
+                Sums<1> e;
+                e.clear();
+#pragma unroll
+                for (int k = 0; k < MT; ++k) e.add_cols(w_lds + m, LD, k, d[k]);
+                const floatx4 z = e.sum(0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (valid) d_enc[(size_t)(m0 + m + 4 * g + r) * N + q] = z[r];
             }
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < UB; ++i)
-#pragma unroll
-                for (int j = 0; j < QB; ++j) acc[i][j] = 0.0f;
-            lds_gemm<W, Q>(wt, bufB, W, u0, q0, acc);
-#pragma unroll
-            for (int i = 0; i < UB; ++i)
-#pragma unroll
-                for (int j = 0; j < QB; ++j) {
-                    const uint32_t m = m0 + u0 + i, q = tq0 + q0 + j;
-                    if (m < K && q < N) d_enc[(size_t)m * N + q] = acc[i][j];
-                }
         }
     }
 }
@@ -290,7 +312,6 @@ __device__ __forceinline__ void wgrad_tile(uint32_t N, const WgradItem& it, uint
                                            const float* __restrict__ A, const float* __restrict__ B,
                                            float* __restrict__ p, uint32_t ld, float4* lds) {
     const int lane = threadIdx.x & 63, g = lane >> 4, m16 = lane & 15, wave = threadIdx.x >> 6;
-    typedef float floatx4 __attribute__((ext_vector_type(4)));
     floatx4 acc[RT * CT];
 #pragma unroll
     for (int t = 0; t < RT * CT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -392,28 +413,13 @@ MlpArgs make_args(const NetShape& n) {
     return MlpArgs{n.n_input, n.n_hidden_layers, n.n_output, n.n_output_padded, n.activation, n.output_activation};
 }
 
-template <int W, int Q>
-size_t smem_bytes() {
-    constexpr int T = Tiling<W, Q>::T;
-    constexpr int R = W > (int)kChunkK ? W : (int)kChunkK;
-    return sizeof(float) * ((size_t)R * T + (size_t)W * T + (size_t)R * W);
-}
+template <int W>
+constexpr size_t kSmemBytes = sizeof(float) * (W + 16) * kLd<W>;
 
-template <int W, int Q, typename Kern>
+template <int W, typename Kern>
 uint32_t grid_for(Kern kern, uint32_t N) {
-    const int occ = occupancy_blocks((const void*)kern, kThreads, smem_bytes<W, Q>());
-    const uint32_t tiles = div_round_up(N, Tiling<W, Q>::T);
-    return std::min<uint32_t>(tiles, (uint32_t)(cu_count() * occ));
-}
-
-// Calls k with the width and the queries per lane that suit N.
-template <typename K>
-void by_tiling(uint32_t W, uint32_t N, K&& k) {
-    by_width(W, [&](auto Wc) {
-        constexpr int Q = kLargeQ<decltype(Wc)::value>;
-        if (Q > 4 && div_round_up(N, 16 * Q) < (uint32_t)cu_count()) k(Wc, std::integral_constant<int, 4>{});
-        else k(Wc, std::integral_constant<int, Q>{});
-    });
+    const int occ = occupancy_blocks((const void*)kern, kThreads, kSmemBytes<W>);
+    return std::min<uint32_t>(div_round_up(N, kTile), (uint32_t)(cu_count() * occ));
 }
 
 uint32_t wgrad_steps(uint32_t N) { return div_round_up(std::max<uint32_t>(N, 1), kWgradQueries); }
@@ -428,11 +434,11 @@ void mlp_forward_f32(hipStream_t stream, const NetShape& net, const float* weigh
                      float* out, float* hidden) {
     if (N == 0) return;
     const MlpArgs a = make_args(net);
-    by_tiling(net.width, N, [&](auto Wc, auto Qc) {
-        constexpr int W = decltype(Wc)::value, Q = decltype(Qc)::value;
-        auto kern = mlp_fwd_kernel<W, Q>;
-        const uint32_t blocks = grid_for<W, Q>(kern, N);
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), (smem_bytes<W, Q>()), stream, N, a, weights, enc, out,
+    by_width(net.width, [&](auto Wc) {
+        constexpr int W = decltype(Wc)::value;
+        auto kern = mlp_fwd_kernel<W>;
+        const uint32_t blocks = grid_for<W>(kern, N);
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), kSmemBytes<W>, stream, N, a, weights, enc, out,
                            hidden);
     });
     NLOD_LAUNCH_CHECK();
@@ -443,11 +449,11 @@ void mlp_backward_delta_f32(hipStream_t stream, const NetShape& net, const float
                             float* d_enc) {
     if (N == 0) return;
     const MlpArgs a = make_args(net);
-    by_tiling(net.width, N, [&](auto Wc, auto Qc) {
-        constexpr int W = decltype(Wc)::value, Q = decltype(Qc)::value;
-        auto kern = mlp_bwd_delta_kernel<W, Q>;
-        const uint32_t blocks = grid_for<W, Q>(kern, N);
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), (smem_bytes<W, Q>()), stream, N, a, weights, hidden, out,
+    by_width(net.width, [&](auto Wc) {
+        constexpr int W = decltype(Wc)::value;
+        auto kern = mlp_bwd_delta_kernel<W>;
+        const uint32_t blocks = grid_for<W>(kern, N);
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), kSmemBytes<W>, stream, N, a, weights, hidden, out,
                            d_out, delta, delta_out, d_enc);
     });
     NLOD_LAUNCH_CHECK();
