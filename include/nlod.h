@@ -350,7 +350,8 @@ int nlod_wavefront_run_thresholds(nlod_wavefront* wavefront, void* stream, uint3
                                   float* d_thr_out, int shape);
 
 /* A sequence of n_batches wavefronts (counts on the host) stored back to back
- * in the buffers.  use_graph: the sequence is captured in a hipGraph on the
+ * in the buffers, run as one batch (a segment's outputs do not depend on its
+ * wavefront).  use_graph: the sequence is captured in a hipGraph on the
  * first call with these sizes and buffers (that call runs eagerly) and
  * replayed by later calls. */
 int nlod_wavefront_run_batches(nlod_wavefront* wavefront, void* stream, uint32_t n_batches, const uint32_t* counts,
