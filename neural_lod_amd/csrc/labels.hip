@@ -351,11 +351,13 @@ struct GroupList {
     }
 };
 
+// Sample i on G lanes; `store`: this group's result is wanted (see the caller).
 template <int G>
 __device__ __forceinline__ void throughput_sample(const LevelsDev& g, const float* __restrict__ tris,
-                                                  const SampleSetup& su, uint64_t i, uint32_t spp, uint32_t max_depth,
-                                                  uint64_t albedo_seed, float* __restrict__ inputs,
-                                                  float* __restrict__ targets, float* __restrict__ valid) {
+                                                  const SampleSetup& su, uint64_t i, bool store, uint32_t spp,
+                                                  uint32_t max_depth, uint64_t albedo_seed,
+                                                  float* __restrict__ inputs, float* __restrict__ targets,
+                                                  float* __restrict__ valid) {
     const int lane = threadIdx.x & 63, sub = lane & (G - 1);
     const LevelDev& L = g.l[su.lod];
     uint64_t st = su.st;
@@ -468,7 +470,7 @@ __device__ __forceinline__ void throughput_sample(const LevelsDev& g, const floa
             ++n_valid;
         }
     }
-    if (sub == 0) {
+    if (store && sub == 0) {
         float* in = inputs + i * 10;
         in[0] = (box.c.x - g.bmin[0]) / (g.bmax[0] - g.bmin[0]);
         in[1] = (box.c.y - g.bmin[1]) / (g.bmax[1] - g.bmin[1]);
@@ -529,28 +531,29 @@ __global__ __launch_bounds__(kLabelThreads, 4) void throughput_samples_kernel(
     const uint32_t n64 = n_of[0], n16 = n_of[1], n4 = n_of[2];
     const uint32_t items16 = (n16 + 3) / 4, items4 = (n4 + 15) / 16;
     for (;;) {
-        // every lane counts, so an item is 64: a branch on the lane here would be
-        // threaded with the one that ends a sample, and lanes would go on alone
+        // The wave's ticket is what its lane 0 gets back: lane 0 adds 1 and the
+        // others 0, so it is the wave's alone in whatever order lanes and waves
+        // add.  A select and not a branch, and groups past the last sample repeat
+        // that sample without storing it: the samples have no branch on the lane
+        // that a wave could leave in parts.
         __builtin_amdgcn_wave_barrier();
-        const uint32_t item = (uint32_t)__builtin_amdgcn_readfirstlane((int)atomicAdd(&next_item, 1u)) / 64u;
+        const uint32_t ticket = atomicAdd(&next_item, lane == 0 ? 1u : 0u);
+        const uint32_t item = (uint32_t)__builtin_amdgcn_readfirstlane((int)ticket);
         if (item >= n64 + items16 + items4) break;
         if (item < n64) {
             const uint32_t sm = order[item];
-            throughput_sample<64>(g, tris, setup[sm], i0 + sm, spp, max_depth, albedo_seed, inputs, targets, valid);
+            throughput_sample<64>(g, tris, setup[sm], i0 + sm, true, spp, max_depth, albedo_seed, inputs, targets,
+                                  valid);
         } else if (item < n64 + items16) {
             const uint32_t k = (item - n64) * 4 + lane / 16;
-            if (k < n16) {
-                const uint32_t sm = order[n64 + k];
-                throughput_sample<16>(g, tris, setup[sm], i0 + sm, spp, max_depth, albedo_seed, inputs, targets,
-                                      valid);
-            }
+            const uint32_t sm = order[n64 + min(k, n16 - 1)];
+            throughput_sample<16>(g, tris, setup[sm], i0 + sm, k < n16, spp, max_depth, albedo_seed, inputs, targets,
+                                  valid);
         } else {
             const uint32_t k = (item - n64 - items16) * 16 + lane / 4;
-            if (k < n4) {
-                const uint32_t sm = order[n64 + n16 + k];
-                throughput_sample<4>(g, tris, setup[sm], i0 + sm, spp, max_depth, albedo_seed, inputs, targets,
-                                     valid);
-            }
+            const uint32_t sm = order[n64 + n16 + min(k, n4 - 1)];
+            throughput_sample<4>(g, tris, setup[sm], i0 + sm, k < n4, spp, max_depth, albedo_seed, inputs, targets,
+                                 valid);
         }
     }
 }

@@ -96,6 +96,24 @@ def test_throughput_block_edges(oracle, cuda, n, spp, max_depth):
     assert np.array_equal(t.cpu().numpy(), et), f"{int((t.cpu().numpy() != et).any(axis=1).sum())} targets differ"
 
 
+@pytest.mark.parametrize("n", [32769, 70001])
+def test_throughput_every_sample_once(cuda, n):
+    """The waves of a block take its samples (32 and 64 of them at these sizes on
+    256 CUs) from one counter: every row is written, with what calls of 777 samples,
+    whose blocks hold 4, write for the same indices.  The last block is not full."""
+    from neural_lod_amd.labels import Labeler
+    tris = S.blob_mesh(20_000, seed=6)
+    print(f"case throughput every sample n={n}", flush=True)
+    lb = Labeler(torch.from_numpy(tris).cuda(), 64, 4)
+    out = tuple(torch.full(shape, float("nan"), device="cuda") for shape in ((n, 10), (n, 3), (n,)))
+    lb.throughput(n, seed=31, first=5, spp=2, max_depth=3, albedo_seed=8, out=out)
+    for first in range(0, n, 777):
+        m = min(777, n - first)
+        part = lb.throughput(m, seed=31, first=5 + first, spp=2, max_depth=3, albedo_seed=8)
+        for whole, p in zip(out, part):
+            assert torch.equal(whole[first:first + m], p), f"samples {first} .. {first + m}"
+
+
 def test_throughput_invalid_arguments(cuda):
     from neural_lod_amd._lib import NlodError
     from neural_lod_amd.labels import Labeler
