@@ -1112,23 +1112,50 @@ __global__ __launch_bounds__(kBboxThreads) void bbox_kernel(const float* __restr
 // Blocks of the bounding-box reduction: two per CU at most.
 uint32_t max_bbox_blocks() { return (uint32_t)cu_count() * 2; }
 
-// The blocks' boxes (6 words each) of the bounding-box reduction, one array per
-// (device, stream), allocated on first use: calls on different streams (from
-// different host threads) never share one, and calls on one stream are ordered
-// by it.
-uint32_t* bbox_blocks(hipStream_t s) {
-    static std::mutex mu;
-    static std::map<std::pair<int, hipStream_t>, std::unique_ptr<DevBuf>> per;
-    int dev = 0;
-    NLOD_HIP(hipGetDevice(&dev));
-    std::lock_guard<std::mutex> lock(mu);
-    auto& b = per[std::make_pair(dev, s)];
-    if (!b) {
-        b.reset(new DevBuf());
-        b->ensure((size_t)max_bbox_blocks() * 6 * sizeof(uint32_t));
+// Device array for the blocks' boxes (6 words each) of one bounding-box call,
+// the call's own from its launch to its wait: a call is two operations, a kernel
+// and a copy, and another thread's call may come between them on the same stream.
+// Up to kMaxSpare arrays are kept for later calls.
+class BboxBlocks {
+public:
+    BboxBlocks() {
+        NLOD_HIP(hipGetDevice(&dev_));
+        {
+            std::lock_guard<std::mutex> lock(mutex());
+            auto& free = spare();
+            for (size_t k = free.size(); k-- > 0 && !buf_;)
+                if (free[k].first == dev_) {
+                    buf_ = std::move(free[k].second);
+                    free.erase(free.begin() + (ptrdiff_t)k);
+                }
+        }
+        if (buf_) return;
+        buf_.reset(new DevBuf());
+        buf_->ensure((size_t)max_bbox_blocks() * 6 * sizeof(uint32_t));
     }
-    return b->as<uint32_t>();
-}
+    BboxBlocks(const BboxBlocks&) = delete;
+    BboxBlocks& operator=(const BboxBlocks&) = delete;
+    uint32_t* get() const { return buf_->as<uint32_t>(); }
+    // The call has waited for its work: the array may serve another one.  Without
+    // this (the call failed) it is freed.
+    void give_back() {
+        std::lock_guard<std::mutex> lock(mutex());
+        if (spare().size() < kMaxSpare) spare().emplace_back(dev_, std::move(buf_));
+    }
+
+private:
+    static constexpr size_t kMaxSpare = 8;
+    static std::mutex& mutex() {
+        static std::mutex m;
+        return m;
+    }
+    static std::vector<std::pair<int, std::unique_ptr<DevBuf>>>& spare() {
+        static std::vector<std::pair<int, std::unique_ptr<DevBuf>>> v;
+        return v;
+    }
+    int dev_ = 0;
+    std::unique_ptr<DevBuf> buf_;
+};
 
 // Tile shape for a G^3 row-major table: T x T rows with T the smallest
 // size >= kMinTile that keeps the tile count within kMaxTileCount (the count
@@ -1389,16 +1416,19 @@ void voxelize(hipStream_t stream, const nlod_voxinfo* info, const float* d_tris,
 
 void mesh_bbox(hipStream_t stream, const float* d_tris, uint64_t n_tri, float bmin[3], float bmax[3]) {
     NLOD_CHECK(n_tri > 0 && d_tris != nullptr, "mesh must have at least one triangle");
-    uint32_t* block_box = bbox_blocks(stream);
+    BboxBlocks block_box;
     const bool aligned16 = (reinterpret_cast<uintptr_t>(d_tris) & 15u) == 0;
     const uint64_t n_vals = n_tri * 9;
     const uint64_t per_block = aligned16 ? 12 * kBboxThreads : kBboxThreads;  // floats per block step
     const uint32_t blocks = (uint32_t)std::min<uint64_t>(div_round_up(n_vals, per_block), max_bbox_blocks());
-    hipLaunchKernelGGL(bbox_kernel, dim3(blocks), dim3(kBboxThreads), 0, stream, d_tris, n_vals, aligned16, block_box);
+    hipLaunchKernelGGL(bbox_kernel, dim3(blocks), dim3(kBboxThreads), 0, stream, d_tris, n_vals, aligned16,
+                       block_box.get());
     NLOD_LAUNCH_CHECK();
     std::vector<uint32_t> boxes((size_t)blocks * 6);
-    NLOD_HIP(hipMemcpyAsync(boxes.data(), block_box, boxes.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
+    NLOD_HIP(hipMemcpyAsync(boxes.data(), block_box.get(), boxes.size() * sizeof(uint32_t), hipMemcpyDeviceToHost,
+                            stream));
     NLOD_HIP(hipStreamSynchronize(stream));
+    block_box.give_back();
     uint32_t h[6] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0u, 0u, 0u};
     for (uint32_t b = 0; b < blocks; ++b)
         for (int d = 0; d < 3; ++d) {

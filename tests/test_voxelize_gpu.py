@@ -179,6 +179,32 @@ def test_mesh_bbox_block_edges(cuda, n_tri, at):
     np.testing.assert_array_equal(mx, v.max(axis=0))
 
 
+def test_mesh_bbox_threads_on_one_stream(cuda):
+    """Threads that ask for the boxes of different meshes on one stream: each gets
+    its own mesh's box, in whatever order their kernels and copies are enqueued."""
+    import threading
+
+    from neural_lod_amd import voxelizer as V
+    sizes = (200_000, 700, 40_000, 1)
+    meshes = [torch.rand((n, 9), device="cuda") * (k + 1) + 10.0 * k for k, n in enumerate(sizes)]
+    want = [(m.view(-1, 3).amin(0).cpu().numpy(), m.view(-1, 3).amax(0).cpu().numpy()) for m in meshes]
+    print("case bbox threads", flush=True)
+    wrong = []
+
+    def ask(k):
+        for _ in range(200):
+            mn, mx = V.mesh_bbox(meshes[k])
+            if not (np.array_equal(mn, want[k][0]) and np.array_equal(mx, want[k][1])):
+                wrong.append(k)
+
+    threads = [threading.Thread(target=ask, args=(k,)) for k in range(len(sizes))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+
+
 @pytest.mark.parametrize("n_tri", [1, 2, 3, 4, 5, 7, 1000, 200_001])
 @pytest.mark.parametrize("offset", [0, 1])
 def test_mesh_bbox(cuda, n_tri, offset):
