@@ -498,7 +498,7 @@ __global__ __launch_bounds__(kLabelThreads, 4) void throughput_samples_kernel(
     __shared__ SampleSetup setup[kMaxBlockSamples];
     __shared__ uint8_t order[kMaxBlockSamples];  // samples on 64 lanes, then on 16, then on 4
     __shared__ uint32_t n_of[3];
-    __shared__ uint32_t next_item;
+    __shared__ uint32_t next_item[64];
     const uint64_t i0 = (uint64_t)blockIdx.x * block_samples;
     const int lane = threadIdx.x & 63;
     if (threadIdx.x < 64) {
@@ -525,19 +525,20 @@ __global__ __launch_bounds__(kLabelThreads, 4) void throughput_samples_kernel(
             at += (uint32_t)__popcll(m);
             if (lane == 0) n_of[c] = (uint32_t)__popcll(m);
         }
-        if (lane == 0) next_item = 0;
+        next_item[lane] = 0;
     }
     __syncthreads();
     const uint32_t n64 = n_of[0], n16 = n_of[1], n4 = n_of[2];
     const uint32_t items16 = (n16 + 3) / 4, items4 = (n4 + 15) / 16;
     for (;;) {
-        // The wave's ticket is what its lane 0 gets back: lane 0 adds 1 and the
-        // others 0, so it is the wave's alone in whatever order lanes and waves
-        // add.  A select and not a branch, and groups past the last sample repeat
-        // that sample without storing it: the samples have no branch on the lane
-        // that a wave could leave in parts.
+        // Every lane adds to a counter of its own and the wave takes what lane 0
+        // gets back, so the ticket is the wave's alone in whatever order lanes and
+        // waves add.  (Lane 0 adding 1 and the others 0 to one counter is as safe,
+        // but becomes a scan over the lanes; 64 counters are one instruction.)  No
+        // branch on the lane, and groups past the last sample repeat that sample
+        // without storing it: nothing here that a wave could leave in parts.
         __builtin_amdgcn_wave_barrier();
-        const uint32_t ticket = atomicAdd(&next_item, lane == 0 ? 1u : 0u);
+        const uint32_t ticket = atomicAdd(&next_item[lane], 1u);
         const uint32_t item = (uint32_t)__builtin_amdgcn_readfirstlane((int)ticket);
         if (item >= n64 + items16 + items4) break;
         if (item < n64) {
