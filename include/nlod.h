@@ -478,10 +478,10 @@ typedef struct nlod_camera {
 } nlod_camera;
 
 enum nlod_tracer_schedule {
-    NLOD_TRACER_AUTO = 0,       /* persistent where it applies, else the reference's (for 128-wide FP16
-                                 * networks: its frame, bit for bit, from one launch) */
+    NLOD_TRACER_AUTO = 0,       /* persistent where it applies, else the reference's */
     NLOD_TRACER_REFERENCE = 1,  /* the reference's wavefront rounds, one host count readback per round */
-    NLOD_TRACER_PERSISTENT = 2  /* FP16: one launch per frame, device ray queue, no host readback */
+    NLOD_TRACER_PERSISTENT = 2  /* FP16: one launch per frame, device ray queue, no host readback; two networks
+                                 * of one width (32, 64 or 128) and feature count */
 };
 
 /* WavefrontNeuralThroughputVisibilityLod parameters

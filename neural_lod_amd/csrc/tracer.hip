@@ -822,7 +822,7 @@ struct Tracer {
     bool wide_ok = false;  // 128-wide FP16 networks: the persistent launch, with the throughput weights in the caches
     uint32_t F = 2, maxdeg = 4;
     size_t smem = 0;  // weights of the persistent launch
-    DevBuf rays_a, rays_b, rays_hit, vis_in, vis_out, thr_in, thr_out, counters, queue, wide_queue;
+    DevBuf rays_a, rays_b, rays_hit, vis_in, vis_out, thr_in, thr_out, counters, queue;
     hipEvent_t ev = nullptr;
     uint32_t* host_counts = nullptr;  // pinned readback of the reference schedule's counters
 
@@ -905,13 +905,13 @@ struct Tracer {
     int pick(const nlod_tracer_params& p) const {
         if (p.schedule == NLOD_TRACER_REFERENCE) return NLOD_TRACER_REFERENCE;
         if (p.schedule == NLOD_TRACER_PERSISTENT) {
-            if (!persistent_ok)
+            if (!persistent_ok && !wide_ok)
                 fail(NLOD_ERR_UNSUPPORTED,
-                     "the persistent schedule needs two FP16 networks of width 32 or 64 with one feature count "
-                     "whose weights fit in LDS");
+                     "the persistent schedule needs two FP16 networks of one width (32, 64 or 128) with one feature "
+                     "count whose weights (at width 128: the visibility network's) fit in LDS");
             return NLOD_TRACER_PERSISTENT;
         }
-        return persistent_ok ? NLOD_TRACER_PERSISTENT : NLOD_TRACER_REFERENCE;
+        return persistent_ok || wide_ok ? NLOD_TRACER_PERSISTENT : NLOD_TRACER_REFERENCE;
     }
 
     void render(hipStream_t s, const nlod_camera& cam, const nlod_tracer_params& p, uint32_t sample_idx,
@@ -920,14 +920,12 @@ struct Tracer {
         vis.require_params(true);
         thr.require_params(true);
         const TracerArgs a = args(cam, p, sample_idx, sample_offset);
-        // AUTO with 128-wide networks gives the reference schedule's frame from one launch
-        if (pick(p) == NLOD_TRACER_PERSISTENT || (wide_ok && p.schedule == NLOD_TRACER_AUTO)) render_persistent(s, a, illum, inferences, bounces);
+        if (pick(p) == NLOD_TRACER_PERSISTENT) render_persistent(s, a, illum, inferences, bounces);
         else render_reference(s, a, illum, inferences, bounces);
     }
 
     void render_persistent(hipStream_t s, const TracerArgs& a, float* illum, uint32_t* inferences,
                            uint32_t* bounces) {
-        DevBuf& queue = wide_ok ? wide_queue : this->queue;  // stats() reports PERSISTENT frames
         queue.ensure(sizeof(uint32_t) * 64);
         const NetArgs av = net_args_of(vis, 0);
         const NetArgs at = net_args_of(thr, wide_ok ? 0 : av.packed_halves);

@@ -198,11 +198,29 @@ def test_reference_networks_width_128(scene):
                                        thr_cfg=configs.REFERENCE_THROUGHPUT)
     tr = TR.Tracer(grid, vis, thr)
     cam = _camera(info, 40, 30)
-    p = TR.default_params(lod=1)
+    p = TR.default_params(lod=1, schedule=TR.REFERENCE)
     assert tr.schedule(p) == TR.REFERENCE
     got = _render(tr, cam, p)
     ref = OT.trace(_oracle_scene(grid, info, 1), OT.camera_from(cam), OT.params_from(p, 9, G), _gpu_net(vis, thr))
     _assert_same(got, ref, "reference networks")
+
+
+def test_wide_networks_schedule_and_statistics(scene):
+    """128-wide networks: AUTO reports the schedule that it renders, PERSISTENT
+    can be asked for, both give one frame, and the statistics are that frame's."""
+    grid, info = scene
+    (vis, _, _), (thr, _, _) = _models(1, seed=17, vis_cfg=configs.REFERENCE_VISIBILITY,
+                                       thr_cfg=configs.REFERENCE_THROUGHPUT)
+    tr = TR.Tracer(grid, vis, thr)
+    cam = _camera(info, 80, 60)
+    auto, asked = TR.default_params(lod=1), TR.default_params(lod=1, schedule=TR.PERSISTENT)
+    assert tr.schedule(auto) == TR.PERSISTENT and tr.schedule(asked) == TR.PERSISTENT
+    print("case wide schedule", flush=True)
+    got = _render(tr, cam, auto)
+    for st in (tr.stats(), (_assert_same(_render(tr, cam, asked), got, "asked for"), tr.stats())[1]):
+        assert st["visibility_queries"] == int(got[1].astype(np.int64).sum())
+        assert st["visibility_tiles"] > 0 and st["wave_rounds"] > 0
+        assert 16 * st["throughput_tiles"] >= st["throughput_queries"] >= st["throughput_tiles"] > 0
 
 
 @pytest.mark.parametrize("name,w,h", [("default", 80, 60), ("hg", 33, 1), ("roulette", 80, 60), ("stochastic", 80, 60),
