@@ -527,7 +527,10 @@ int nlod_tracer_destroy(nlod_tracer* tracer);
  * uint32[width * height] its visibility-network queries (needed_inferences),
  * d_bounces (nullable) the bounce at which it ended.  The reference schedule
  * synchronizes the stream once per round; the persistent one is asynchronous,
- * allocates nothing after its first call and can be captured in a hipGraph. */
+ * allocates nothing after its first call and can be captured in a hipGraph.
+ * Persistent frames of one tracer may be in flight on several streams; replays
+ * of a captured one must be ordered by the caller with the tracer's other frames
+ * on the stream that it was captured on, and with other captured frames. */
 int nlod_tracer_render(nlod_tracer* tracer, void* stream, const nlod_camera* camera,
                        const nlod_tracer_params* params, uint32_t sample_idx, uint32_t sample_offset,
                        float* d_illumination, uint32_t* d_inferences, uint32_t* d_bounces);
@@ -535,8 +538,8 @@ int nlod_tracer_render(nlod_tracer* tracer, void* stream, const nlod_camera* cam
  * network evaluations (one per 16-slot tile of a wave), [1] the visibility
  * queries they served, [2] and [3] the same for the throughput network, [4]
  * the waves' rounds.  [1] / (16 [0]) is the tile occupancy of the network
- * evaluations.  Synchronizes the stream; zeros before the first persistent
- * frame.  No counterpart in the reference. */
+ * evaluations.  Synchronizes the stream (the device, when that frame was enqueued
+ * on another one); zeros before the first persistent frame.  No counterpart in the reference. */
 int nlod_tracer_stats(nlod_tracer* tracer, void* stream, uint64_t stats_out[5]);
 /* The schedule nlod_tracer_render would use for these parameters. */
 int nlod_tracer_schedule(const nlod_tracer* tracer, const nlod_tracer_params* params, int* schedule_out);

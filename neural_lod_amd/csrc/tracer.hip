@@ -823,7 +823,18 @@ struct Tracer {
     uint32_t F = 2, maxdeg = 4;
     size_t smem = 0;  // weights of the persistent launch
     DevBuf rays_a, rays_b, rays_hit, vis_in, vis_out, thr_in, thr_out, counters, queue;
-    hipEvent_t ev = nullptr;
+    // Persistent frames of different streams may run at once, so each stream has a
+    // ray queue of its own, up to kQueues of them (an event between the frames cost
+    // 5 us a frame, 225 us for 64 x 64 paths).  The least recently used one goes to
+    // another stream when the device has nothing left to do on it.
+    static constexpr int kQueues = 16, kQueueWords = 64;
+    struct StreamQueue {
+        hipStream_t stream;
+        uint64_t last_use;  // 0: free
+    };
+    StreamQueue queues[kQueues] = {};
+    int last_queue = -1;  // of the last persistent frame
+    uint64_t frames = 0;
     uint32_t* host_counts = nullptr;  // pinned readback of the reference schedule's counters
 
     Tracer(const LodGrid& g, Model& v, Model& t) : grid(g), vis(v), thr(t) {
@@ -848,11 +859,9 @@ struct Tracer {
             wide_ok = smem + rows_bytes(kTraceBlock) <= kMaxTraceLds;
         }
         NLOD_HIP(hipHostMalloc((void**)&host_counts, 4 * sizeof(uint32_t), hipHostMallocDefault));
-        NLOD_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     }
     ~Tracer() {
         if (host_counts) (void)hipHostFree(host_counts);
-        if (ev) (void)hipEventDestroy(ev);
     }
 
     // network inputs and outputs of a block's ray slots
@@ -924,12 +933,33 @@ struct Tracer {
         else render_reference(s, a, illum, inferences, bounces);
     }
 
+    uint32_t* queue_of(hipStream_t s) {
+        queue.ensure(sizeof(uint32_t) * kQueues * kQueueWords);
+        int at = 0;
+        for (int k = 0; k < kQueues; ++k) {
+            if (queues[k].last_use && queues[k].stream == s) {
+                at = k;
+                break;
+            }
+            if (queues[k].last_use < queues[at].last_use) at = k;
+        }
+        if (queues[at].last_use && queues[at].stream != s) {
+            // a captured frame runs when its graph is launched: the caller orders it
+            hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+            NLOD_HIP(hipStreamIsCapturing(s, &capturing));
+            if (capturing == hipStreamCaptureStatusNone) NLOD_HIP(hipDeviceSynchronize());
+        }
+        queues[at] = {s, ++frames};
+        last_queue = at;
+        return queue.as<uint32_t>() + at * kQueueWords;
+    }
+
     void render_persistent(hipStream_t s, const TracerArgs& a, float* illum, uint32_t* inferences,
                            uint32_t* bounces) {
-        queue.ensure(sizeof(uint32_t) * 64);
+        uint32_t* const rays = queue_of(s);
         const NetArgs av = net_args_of(vis, 0);
         const NetArgs at = net_args_of(thr, wide_ok ? 0 : av.packed_halves);
-        hipLaunchKernelGGL(reset_queue_kernel, dim3(1), dim3(64), 0, s, queue.as<uint32_t>());
+        hipLaunchKernelGGL(reset_queue_kernel, dim3(1), dim3(64), 0, s, rays);
         NLOD_LAUNCH_CHECK();
         const size_t bits_bytes = sizeof(uint32_t) * (((size_t)a.R * a.R * a.R + 31) / 32);
         auto by_block = [&](auto Wc, auto Fc, auto Dc, auto Bc) {
@@ -952,8 +982,7 @@ struct Tracer {
             al.slots = std::min<uint32_t>(kSlots, div_round_up(a.n_rays, blocks * (block / 64)));
             hipLaunchKernelGGL(kern, dim3(blocks), dim3(block), launch_smem, s, al, av, at,
                                static_cast<const half_t*>(vis.packed_fwd(true)),
-                               static_cast<const half_t*>(thr.packed_fwd(true)), queue.as<uint32_t>(), illum,
-                               inferences, bounces);
+                               static_cast<const half_t*>(thr.packed_fwd(true)), rays, illum, inferences, bounces);
         };
         using Block = std::integral_constant<int, kTraceBlock>;
         using BlockSmall = std::integral_constant<int, kTraceBlockSmall>;
@@ -973,8 +1002,10 @@ struct Tracer {
     // statistics of the last persistent frame (synchronizes the stream)
     void stats(hipStream_t s, uint64_t* out) {
         std::memset(out, 0, 5 * sizeof(uint64_t));
-        if (!queue.p) return;
-        NLOD_HIP(hipMemcpyAsync(out, queue.as<uint32_t>() + 16, 5 * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+        if (last_queue < 0) return;
+        if (queues[last_queue].stream != s) NLOD_HIP(hipDeviceSynchronize());
+        NLOD_HIP(hipMemcpyAsync(out, queue.as<uint32_t>() + last_queue * kQueueWords + 16, 5 * sizeof(uint64_t),
+                                hipMemcpyDeviceToHost, s));
         NLOD_HIP(hipStreamSynchronize(s));
     }
 

@@ -242,6 +242,38 @@ def test_wide_networks_one_launch_equals_rounds(scene, name, w, h):
     assert (got[1] >= 1).any()
 
 
+@pytest.mark.parametrize("width,n_streams", [(64, 2), (128, 2), (128, 19)])
+def test_frames_of_one_tracer_on_several_streams(scene, width, n_streams):
+    """Frames of one tracer enqueued on several streams without a wait between them
+    must each be the frame rendered alone, also on more streams than the tracer has
+    ray queues (16), and the statistics the last one's."""
+    grid, info = scene
+    nets = {} if width == 64 else {"vis_cfg": configs.REFERENCE_VISIBILITY, "thr_cfg": configs.REFERENCE_THROUGHPUT}
+    (vis, _, _), (thr, _, _) = _models(1, seed=23, **nets)
+    tr = TR.Tracer(grid, vis, thr)
+    p = TR.default_params(lod=1, schedule=TR.PERSISTENT)
+    cams = [_camera(info, 300, 200), _camera(info, 64, 40), _camera(info, 101, 77)]
+    alone = [_render(tr, c, p, k) for k, c in enumerate(cams)]
+    print(f"case streams width={width} n={n_streams}", flush=True)
+    streams = [torch.cuda.Stream() for _ in range(n_streams)]
+    main = torch.cuda.current_stream()
+    outs = []
+    for rep in range(3):
+        for k, s in enumerate(streams):
+            out = tuple(torch.empty_like(torch.from_numpy(t.view(np.int32) if t.dtype == np.uint32 else t),
+                                         device="cuda") for t in alone[k % 3])
+            s.wait_stream(main)
+            with torch.cuda.stream(s):
+                outs.append((k % 3, tr.render(cams[k % 3], p, sample_idx=k % 3, out=out)))
+    with torch.cuda.stream(streams[0]):
+        st = tr.stats()
+    torch.cuda.synchronize()
+    for k, out in outs:
+        illum, inf, bnc = (t.cpu().numpy() for t in out)
+        _assert_same((illum, inf.view(np.uint32), bnc.view(np.uint32)), alone[k], f"frame {k}")
+    assert st["visibility_queries"] == int(alone[(n_streams - 1) % 3][1].astype(np.int64).sum())
+
+
 def test_persistent_graph_replays(scene):
     grid, info = scene
     (vis, _, _), (thr, _, _) = _models(1, seed=5)
