@@ -1,6 +1,6 @@
 // FP16-MFMA form of the encode + fully fused MLP (gfx950).
 //
-// Three launches per batch, two below kLdsFrom queries (without 0.):
+// Three launches per batch, two for smaller ones (without 0., see lds_pass_pays):
 //  0. The coarse levels whose FP16 tables fit in LDS together (72 KB: levels 0
 //     and 1 of the 16^3-based grids): encode_lds_kernel gathers from a copy of
 //     those tables in LDS, sparing the L2 that the other levels saturate.
@@ -410,38 +410,66 @@ __global__ void to_half_kernel(const float* __restrict__ src, half_t* __restrict
         dst[i] = (half_t)src[i];
 }
 
-// Batches from which the LDS pass pays.  It costs a launch whose blocks each copy
-// 70 KB first, 7 us at any size, and spares the level rows 2 of 14 tables: 64-wide
-// networks, 1793 queries 16.9 us with it and 9.8 without, 131072 61.3 and 56.4,
-// 262144 97.7 and 97.3, 524288 199 and 205; 144-input 128-wide one, 265621 queries
-// 93.2 and 89.6.
-constexpr uint32_t kLdsFrom = 300000;
+// True when every grid segment reads the same 3 inputs, from offset `off`.
+bool one_position(const Layout& L, uint32_t& off) {
+    bool any = false;
+    for (const Segment& s : L.segs) {
+        if (s.type != SEG_GRID) continue;
+        if (any && s.in_offset != off) return false;
+        off = s.in_offset;
+        any = true;
+    }
+    return any;
+}
+
+// Whether the LDS pass pays for a batch of N queries.  It is a launch whose blocks
+// each copy up to 72 KB first, about 7 us at any size.  It spares the level rows
+// its own levels, and all the others the reading of positions from the queries'
+// rows when they take them from its [3][N] copy; the weight of a level in LDS
+// against a byte of such reads, and the total, fit the queries at which both forms
+// take equally long (kernels alone; 16 levels in 6 inputs 340,000, 9 inputs 210,000,
+// 10 inputs 178,000, 14 inputs 105,000; 8 levels in 6 inputs 430,000, 10 inputs
+// 340,000; 7 levels in 9 inputs 350,000; two positions of 7 levels 370,000).  16 levels, 6
+// inputs: 100,000 queries 48 us with the pass and 43 without, 500,000 149 and 153;
+// 10 inputs: 50 and 47, 157 and 168.
+bool lds_pass_pays(const Layout& L, uint32_t N, uint32_t n_lds, uint32_t n_rows) {
+    uint32_t off = 0;
+    uint64_t spared = 90ull * n_lds;
+    if (one_position(L, off)) spared += (uint64_t)n_rows * sizeof(float) * L.n_input_dims;
+    return N * spared >= 136000000ull;
+}
 
 // Splits the grid levels between the LDS pass (levels whose tables still fit,
 // in order) and the rows of the per-level pass (the rest; all levels of a batch
-// of N < kLdsFrom queries).
+// that is too small for the LDS pass).
 void make_level_maps(const Layout& L, uint32_t N, LevelMap& m, LdsLevels& d) {
-    m = LevelMap{};
-    d = LdsLevels{};
-    for (size_t si = 0; si < L.segs.size(); ++si) {
-        const Segment& s = L.segs[si];
-        if (s.type != SEG_GRID) continue;
-        for (uint32_t l = 0; l < s.n_levels; ++l) {
-            const uint32_t halves = (s.levels.offset[l + 1] - s.levels.offset[l]) * s.F;
-            if (N >= kLdsFrom && d.n < (uint32_t)kMaxLdsLevels && (size_t)(d.halves + halves) * sizeof(half_t) <= kLdsTableBytes) {
-                d.seg[d.n] = (uint8_t)si;
-                d.level[d.n] = (uint8_t)l;
-                d.at[d.n] = d.halves;
-                d.halves += halves;
-                ++d.n;
-                continue;
+    auto split = [&](bool use_lds) {
+        m = LevelMap{};
+        d = LdsLevels{};
+        for (size_t si = 0; si < L.segs.size(); ++si) {
+            const Segment& s = L.segs[si];
+            if (s.type != SEG_GRID) continue;
+            for (uint32_t l = 0; l < s.n_levels; ++l) {
+                const uint32_t halves = (s.levels.offset[l + 1] - s.levels.offset[l]) * s.F;
+                if (use_lds && d.n < (uint32_t)kMaxLdsLevels &&
+                    (size_t)(d.halves + halves) * sizeof(half_t) <= kLdsTableBytes) {
+                    d.seg[d.n] = (uint8_t)si;
+                    d.level[d.n] = (uint8_t)l;
+                    d.at[d.n] = d.halves;
+                    d.halves += halves;
+                    ++d.n;
+                    continue;
+                }
+                if (m.n >= (uint32_t)kMaxLevelRows) fail(NLOD_ERR_UNSUPPORTED, "more than 64 grid levels in one model");
+                m.seg[m.n] = (uint8_t)si;
+                m.level[m.n] = (uint8_t)l;
+                ++m.n;
             }
-            if (m.n >= (uint32_t)kMaxLevelRows) fail(NLOD_ERR_UNSUPPORTED, "more than 64 grid levels in one model");
-            m.seg[m.n] = (uint8_t)si;
-            m.level[m.n] = (uint8_t)l;
-            ++m.n;
         }
-    }
+    };
+    const bool may_pay = lds_pass_pays(L, N, kMaxLdsLevels, kMaxLevelRows);
+    split(may_pay);
+    if (may_pay && !lds_pass_pays(L, N, d.n, m.n)) split(false);
 }
 
 }  // namespace
@@ -479,15 +507,8 @@ size_t mfma_pos_scratch_bytes(const Layout& L, uint32_t N) {
     LevelMap map;
     LdsLevels lds;
     make_level_maps(L, N, map, lds);
-    bool any = false, same = true;
     uint32_t off = 0;
-    for (const Segment& s : L.segs) {
-        if (s.type != SEG_GRID) continue;
-        if (any && s.in_offset != off) same = false;
-        off = s.in_offset;
-        any = true;
-    }
-    if (!lds.n || !any || !same || map.n == 0) return 0;
+    if (!lds.n || map.n == 0 || !one_position(L, off)) return 0;
     return sizeof(float) * 3 * (size_t)(div_round_up(N, 16) * 16);
 }
 
@@ -504,8 +525,7 @@ void mfma_encode(hipStream_t stream, const Layout& L, const void* d_program, con
     uint32_t soa_off = 0;
     if (pos_scratch && mfma_pos_scratch_bytes(L, N) > 0) {
         xsoa = static_cast<float*>(pos_scratch);
-        for (const Segment& s : L.segs)
-            if (s.type == SEG_GRID) soa_off = s.in_offset;
+        one_position(L, soa_off);
     }
     if (lds.n) {
         const size_t smem = (size_t)lds.halves * sizeof(half_t);

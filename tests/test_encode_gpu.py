@@ -1,6 +1,7 @@
-"""The FP16 encoding's two forms give the same features, bit for bit: batches of
-300000 queries and more encode the coarse levels from tables in LDS, smaller ones
-take every level row by row."""
+"""The FP16 encoding's two forms give the same features, bit for bit: large batches
+encode the coarse levels from tables in LDS (from 263566 queries of the visibility
+network, 183784 of the throughput network, 377778 of the two-point visibility
+network), smaller ones take every level row by row."""
 import pytest
 import torch
 
@@ -10,8 +11,10 @@ from neural_lod_amd.tcnn import FP16, NetworkWithInputEncoding
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [299999, 300000, 300017])
-@pytest.mark.parametrize("name", ["visibility", "throughput", "reference_visibility"])
+@pytest.mark.parametrize("name,n", [
+    *((name, n) for name in ("visibility", "throughput", "reference_visibility") for n in (299999, 300000, 300017)),
+    ("visibility", 263565), ("visibility", 263566), ("throughput", 183783), ("throughput", 183784),
+    ("reference_visibility", 377777), ("reference_visibility", 377778), ("reference_visibility", 400001)])
 def test_large_batch_features_equal_small_batches(cuda, name, n):
     cfg = configs.ALL[name]
     net = NetworkWithInputEncoding(cfg["n_input_dims"], cfg["n_output_dims"], cfg["encoding"], cfg["network"], FP16)
