@@ -144,11 +144,11 @@ __global__ __launch_bounds__(kFwdThreads<W>) void mlp_fwd_train_kernel(TrainArgs
     }
 }
 
-// LDSW: the weights are staged in LDS (whenever they fit); otherwise every wave
-// reads them from the caches for each of its tiles.  101003 queries of the
-// 144-input 128 x 4 network: 134 us with weights from the caches and 2-byte
-// accesses to H and D, 93 us now (forward with saved activations: 58 -> 42 us).
-template <int W, bool LDSW>
+// The weights are staged in LDS, where they always fit (see mfma_mlp_backward).
+// 101003 queries of the 144-input 128 x 4 network: 134 us with weights from the
+// caches and 2-byte accesses to H and D, 93 us now (forward with saved
+// activations: 58 -> 42 us).
+template <int W>
 __global__ __launch_bounds__(kFwdThreads<W>) void mlp_bwd_kernel(TrainArgs a, const half_t* __restrict__ packed_bwd,
                                                                  const half_t* __restrict__ H,
                                                                  const float* __restrict__ y,
@@ -156,12 +156,9 @@ __global__ __launch_bounds__(kFwdThreads<W>) void mlp_bwd_kernel(TrainArgs a, co
                                                                  float* __restrict__ d_enc) {
     constexpr int MT = W / 16, KC = W / 32, NT = kFwdThreads<W>;
     extern __shared__ float4 smem4[];
-    const half_t* sw = packed_bwd;
-    if constexpr (LDSW) {
-        stage_weights<NT>(reinterpret_cast<half_t*>(smem4), packed_bwd, a.packed_bwd_halves);
-        sw = reinterpret_cast<half_t*>(smem4);
-        __syncthreads();
-    }
+    half_t* sw = reinterpret_cast<half_t*>(smem4);
+    stage_weights<NT>(sw, packed_bwd, a.packed_bwd_halves);
+    __syncthreads();
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
     const uint32_t n_tiles = (a.N + 15) / 16;
     const uint32_t n_waves = gridDim.x * (NT / 64);
@@ -418,11 +415,16 @@ void mfma_mlp_backward(hipStream_t stream, const Layout& L, const void* packed_b
                        const float* y, const float* dy, uint32_t N, void* delta, float* d_enc) {
     if (N == 0) return;
     const TrainArgs a = make_targs(L, N);
+    // mfma_supported holds the forward packing to 160 KB, that is to 160 fragments
+    // of 1 KB.  The backward packing has W / 32 fragments more (W / 16 for the
+    // output matrix instead of W / 32); without the output matrix both have a
+    // multiple of W / 16, so that at most 160 - W / 16 of the forward packing's 160
+    // are the shared ones, and the backward packing fits as well.
+    const size_t smem = mfma_packed_bwd_bytes(L.net);
+    if (smem > kMaxLds) fail(NLOD_ERR_UNSUPPORTED, "the backward weights do not fit in LDS");
     by_w(L.net.width, [&](auto Wc) {
         constexpr int W = decltype(Wc)::value;
-        const bool lds = mfma_packed_bwd_bytes(L.net) <= kMaxLds;
-        const size_t smem = lds ? mfma_packed_bwd_bytes(L.net) : 0;
-        auto kern = lds ? mlp_bwd_kernel<W, true> : mlp_bwd_kernel<W, false>;
+        auto kern = mlp_bwd_kernel<W>;
         const uint32_t blocks = persistent_blocks(kern, kFwdThreads<W>, smem, div_round_up(N, 16));
         hipLaunchKernelGGL(kern, dim3(blocks), dim3(kFwdThreads<W>), smem, stream, a, static_cast<const half_t*>(packed_bwd),
                            static_cast<const half_t*>(hidden), y, dy, static_cast<half_t*>(delta), d_enc);
