@@ -1,4 +1,4 @@
-"""FP32 network passes at the edges of their tiles (16 or 32 queries per wave, 4
+"""FP32 network passes at the edges of their tiles (16 queries per wave, 4
 waves per block; 64 columns of the first matrix at a time), against float64.
 
 Every value is a sum of K or W products of FP32 values, layer after layer, so
