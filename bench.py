@@ -124,7 +124,7 @@ def wavefront_bench(dev, args):
             nets.append((m, p))
         wf = Wavefront(nets[0][0], nets[1][0], 0.5)
         if prec == FP16:
-            wf.tune(max(counts))
+            wf.tune(total)
         vo = torch.empty((total, 1), device=dev)
         to = torch.empty((total, 3), device=dev)
         use_graph = prec == FP16

@@ -323,8 +323,10 @@ int nlod_wavefront_create(nlod_model* visibility, nlod_model* throughput, float 
 int nlod_wavefront_destroy(nlod_wavefront* wavefront);
 
 /* Autotuner: times the launch shapes (split launches; fused kernel with 1..max
- * blocks per CU) once per wavefront-size bucket up to max_n queries and keeps
- * the fastest.  Synchronizes the stream.  Untuned engines use the fused kernel
+ * blocks per CU) once per wavefront-size bucket up to max_n queries, with half of
+ * the segments visible, and keeps the fastest.  max_n: the largest wavefront, or
+ * the largest sum of a sequence, which runs as one; larger ones take the choice
+ * made at max_n.  Synchronizes the stream.  Untuned engines use the fused kernel
  * at 1 block per CU where it applies. */
 int nlod_wavefront_tune(nlod_wavefront* wavefront, void* stream, uint32_t max_n);
 /* The shape the engine picks for n queries (0 = split launches, k = fused kernel, k blocks per CU). */

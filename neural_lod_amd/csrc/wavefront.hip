@@ -25,6 +25,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <cmath>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -156,7 +157,11 @@ __global__ __launch_bounds__(kSelectBlock) void select_kernel(uint32_t N, uint32
     }
 }
 static_assert(kSelectPerThread * (kSelectBlock / 64) == 64, "one wave scans the counts");
-constexpr uint32_t kSelectFrom = 16384;  // segments from which the list pays
+// Segments from which the list pays.  Half of them visible, without and with the
+// list, 64-wide networks: 8192 32.6 and 35.3 us, 16384 44.0 and 42.3, 32768 60.1 and
+// 56.7, 2^20 749 and 593; 128-wide: 34.4 and 38.0, 39.3 and 40.6, 50.9 and 48.1, 629
+// and 495.  All visible, 64-wide: 16384 43.6 and 48.6, 2^20 745 and 755.
+constexpr uint32_t kSelectFrom = 16384;
 
 // wavefront-size buckets of the autotuner: [2^k, 2^(k+2)) for k = 8, 10, ..., 20
 constexpr int kBuckets = 8;
@@ -179,7 +184,7 @@ struct Wavefront {
     int choice[kBuckets];
     bool tuned = false;
     int max_blocks_per_cu = 1;
-    DevBuf tune_in_v, tune_in_t, tune_out_v, tune_out_t;
+    DevBuf tune_in_v, tune_in_t, tune_thr, tune_out_v, tune_out_t;
     // visible segments of one pass of the split launches and their number; of
     // full size from the start, so captured sequences may hold its address
     DevBuf selected;
@@ -287,7 +292,10 @@ struct Wavefront {
         else run_split(s, N, vin, tin, vout, tout, seg_thr);
     }
 
-    // Times each candidate once per bucket (synchronizes the stream).
+    // Times each candidate once per bucket (synchronizes the stream), with every
+    // other segment visible: the split form's time depends on that share (2^20
+    // segments: 372 us with none visible, 593 with half, 755 with all).  Buckets
+    // above max_n are timed at max_n.
     void tune(hipStream_t s, uint32_t max_n) {
         if (!fp16 || !fused_ok) {
             tuned = true;
@@ -297,13 +305,16 @@ struct Wavefront {
         const uint32_t nv = vis.L.n_input_dims, nt = thr.L.n_input_dims;
         tune_in_v.ensure(sizeof(float) * (size_t)max_n * nv);
         tune_in_t.ensure(sizeof(float) * (size_t)max_n * nt);
+        tune_thr.ensure(sizeof(float) * (size_t)max_n);
         tune_out_v.ensure(sizeof(float) * (size_t)max_n * vis.L.net.n_output);
         tune_out_t.ensure(sizeof(float) * (size_t)max_n * thr.L.net.n_output);
-        // inputs in [0, 1) from a fixed pattern (any in-range values exercise the same work)
+        // inputs in [0, 1) from a fixed pattern; thresholds that all outputs reach, or none
         std::vector<float> h(std::max<size_t>((size_t)max_n * nv, (size_t)max_n * nt));
         for (size_t i = 0; i < h.size(); ++i) h[i] = (float)((i * 2654435761ull) % 1000003ull) / 1000003.0f;
         NLOD_HIP(hipMemcpy(tune_in_v.p, h.data(), sizeof(float) * (size_t)max_n * nv, hipMemcpyHostToDevice));
         NLOD_HIP(hipMemcpy(tune_in_t.p, h.data(), sizeof(float) * (size_t)max_n * nt, hipMemcpyHostToDevice));
+        for (uint32_t i = 0; i < max_n; ++i) h[i] = i & 1 ? INFINITY : -INFINITY;
+        NLOD_HIP(hipMemcpy(tune_thr.p, h.data(), sizeof(float) * (size_t)max_n, hipMemcpyHostToDevice));
         hipEvent_t e0, e1;
         NLOD_HIP(hipEventCreate(&e0));
         NLOD_HIP(hipEventCreate(&e1));
@@ -314,9 +325,9 @@ struct Wavefront {
             for (int c = 0; c <= max_blocks_per_cu; ++c) {
                 auto launch = [&] {
                     if (c == 0) run_split(s, n, tune_in_v.as<float>(), tune_in_t.as<float>(), tune_out_v.as<float>(),
-                                          tune_out_t.as<float>());
+                                          tune_out_t.as<float>(), tune_thr.as<float>());
                     else run_fused(s, n, tune_in_v.as<float>(), tune_in_t.as<float>(), tune_out_v.as<float>(),
-                                   tune_out_t.as<float>(), c);
+                                   tune_out_t.as<float>(), c, tune_thr.as<float>());
                 };
                 launch();  // warm
                 const int reps = 5;
