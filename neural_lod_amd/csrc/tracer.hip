@@ -583,7 +583,7 @@ __global__ __launch_bounds__(kStageThreads) void bounce_compact_kernel(TracerArg
 
 // ------------------------------------------------------ persistent schedule
 constexpr int kTraceBlock = 768;
-constexpr int kTraceBlockSmall = 512;  // 128-wide networks, frames that this many threads per CU hold at once
+constexpr int kTraceBlockSmall = 512;  // 128-wide networks, small frames (wide_small_block)
 constexpr int kSlots = 64;     // rays in flight per wave at most: one per lane
 // A wave with few rays left evaluates up to this many voxels ahead of each: a
 // tile has 16 rows either way, and the frame ends with the longest ray, whose
@@ -608,10 +608,8 @@ __device__ __forceinline__ uint32_t lane_rank(uint64_t mask) {
 // voxel of a path needs; the throughput network, at most once a bounce, reads
 // its weights from the caches.  480 x 270 paths, 64^3 level, up to 3 bounces:
 // 11.3 ms in the reference schedule (two hundred rounds of a few rays, each nine
-// launches and a host readback), 2.7 ms in this one launch.  12 waves per CU
-// suit large frames (1024 x 1024: 7.6 ms, 8.7 ms with 8), 8 waves those whose
-// rays they hold at once (2.74 against 2.86 ms), which wait for single rays
-// (these times without the voxels ahead, kMaxAhead).
+// launches and a host readback), 2.7 ms in this one launch, 1.6 ms with the voxels
+// ahead (kMaxAhead).
 template <int W, int F, int MAXD, bool LB, int BLOCK>
 __global__ __launch_bounds__(BLOCK, BLOCK / 256) void trace_persistent_kernel(
     TracerArgs a, NetArgs vis, NetArgs thr, const half_t* __restrict__ packed_vis,
@@ -807,6 +805,19 @@ __global__ __launch_bounds__(BLOCK, BLOCK / 256) void trace_persistent_kernel(
     }
 }
 
+// Blocks of 8 waves instead of 12 for 128-wide networks.  The waves of a CU hold each
+// other up when each has a ray or two (64 x 64 paths at 32^3, one bounce: 222 us with
+// 8, 303 with 12); with more bounces, the loads of the throughput weights, which more
+// waves hide, outweigh that for all but the smallest frames.  64^3 level, us with 8
+// and 12 waves: 3 bounces, 128 x 96 746 and 768, 160 x 90 842 and 808, 480 x 270 1702
+// and 1607, 1024 x 1024 7020 and 5950; 2 bounces, 160 x 90 667 and 686, 200 x 120 753
+// and 738, 480 x 270 1297 and 1175.  A single bounce never evaluates the throughput
+// network: 160 x 90 313 and 352, 320 x 180 518 and 534, 480 x 270 745 and 741 (at 32^3
+// 604 and 623).
+inline bool wide_small_block(const TracerArgs& a) {
+    return a.n_rays <= (uint32_t)cu_count() * (a.max_depth == 1 ? kTraceBlockSmall : 56);
+}
+
 // queue[0]: next ray; queue[16 ..]: the frame's statistics (uint64 each)
 __global__ void reset_queue_kernel(uint32_t* q) {
     if (threadIdx.x < 64) q[threadIdx.x] = 0;
@@ -989,7 +1000,7 @@ struct Tracer {
         if (wide_ok) {
             dispatch_wf(32, F, maxdeg, [&](auto, auto Fc, auto Dc) {
                 constexpr std::integral_constant<int, 128> Wc{};
-                if (a.n_rays <= (uint32_t)(cu_count() * kTraceBlockSmall)) by_block(Wc, Fc, Dc, BlockSmall{});
+                if (wide_small_block(a)) by_block(Wc, Fc, Dc, BlockSmall{});
                 else by_block(Wc, Fc, Dc, Block{});
             });
         } else {

@@ -102,6 +102,7 @@ OPTIONS = {
     "lod0": {"lod": 0, "max_depth": 2},
     "lod2": {"lod": 2},
 }
+ONE_BOUNCE = {"one_bounce": {"max_depth": 1}}
 
 
 @pytest.mark.parametrize("name", list(OPTIONS))
@@ -224,17 +225,19 @@ def test_wide_networks_schedule_and_statistics(scene):
 
 
 @pytest.mark.parametrize("name,w,h", [("default", 80, 60), ("hg", 33, 1), ("roulette", 80, 60), ("stochastic", 80, 60),
-                                      ("log_learning", 80, 60), ("lod0", 41, 30), ("lod2", 400, 400)])
+                                      ("log_learning", 80, 60), ("lod0", 41, 30), ("lod2", 400, 400),
+                                      ("default", 128, 112), ("default", 129, 112), ("one_bounce", 129, 112),
+                                      ("one_bounce", 400, 400)])
 def test_wide_networks_one_launch_equals_rounds(scene, name, w, h):
     """128-wide networks: the one launch that AUTO takes against the reference
-    schedule's rounds, bit for bit; frames below and above the block-size switch
-    (131072 rays), levels whose occupancy words fit in LDS (lod2) and do not."""
+    schedule's rounds, bit for bit; frames below and above the block-size switches
+    (14336 rays, 131072 with one bounce), levels whose occupancy words fit in LDS (lod2) and do not."""
     grid, info = scene
     (vis, _, _), (thr, _, _) = _models(1, seed=17, vis_cfg=configs.REFERENCE_VISIBILITY,
                                        thr_cfg=configs.REFERENCE_THROUGHPUT)
     tr = TR.Tracer(grid, vis, thr)
     cam = _camera(info, w, h)
-    kw = dict({"lod": 1, "max_depth": 3}, **OPTIONS[name])
+    kw = dict({"lod": 1, "max_depth": 3}, **{**OPTIONS, **ONE_BOUNCE}[name])
     print(f"case wide frame {name} {w}x{h}", flush=True)
     got = _render(tr, cam, TR.default_params(**kw), 3)
     ref = _render(tr, cam, TR.default_params(schedule=TR.REFERENCE, **kw), 3)
