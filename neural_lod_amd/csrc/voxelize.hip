@@ -1195,22 +1195,32 @@ bool tile_geometry(uint32_t G, uint64_t n_tri, bool force, bool accumulate, Tile
 constexpr size_t kMiscWords = 16;
 
 // Tiled-path scratch, one grow-only buffer per (device, stream); a new
-// buffer's job counters are cleared on the stream before its first job.
-uint8_t* tile_workspace(hipStream_t s, size_t bytes) {
+// buffer's job counters are cleared on the stream before its first job.  `mu` is
+// held while a job's launches are enqueued: another thread's launches on the same
+// stream must not come between them.
+struct TileScratch {
+    std::mutex mu;
+    DevBuf buf;
+    uint8_t* ensure(hipStream_t s, size_t bytes) {
+        if (buf.bytes < bytes) {
+            NLOD_HIP(hipStreamSynchronize(s));  // earlier calls on this stream may still read it
+            buf.ensure(bytes);
+            hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(64), 0, s, buf.as<uint32_t>(), (uint64_t)kMiscWords, 1);
+            NLOD_LAUNCH_CHECK();
+        }
+        return buf.as<uint8_t>();
+    }
+};
+
+TileScratch& tile_scratch(hipStream_t s) {
     static std::mutex mu;
-    static std::map<std::pair<int, hipStream_t>, std::unique_ptr<DevBuf>> per;
+    static std::map<std::pair<int, hipStream_t>, std::unique_ptr<TileScratch>> per;
     int dev = 0;
     NLOD_HIP(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lock(mu);
     auto& b = per[std::make_pair(dev, s)];
-    if (!b) b.reset(new DevBuf());
-    if (b->bytes < bytes) {
-        NLOD_HIP(hipStreamSynchronize(s));  // earlier calls on this stream may still read it
-        b->ensure(bytes);
-        hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(64), 0, s, b->as<uint32_t>(), (uint64_t)kMiscWords, 1);
-        NLOD_LAUNCH_CHECK();
-    }
-    return b->as<uint8_t>();
+    if (!b) b.reset(new TileScratch());
+    return *b;
 }
 
 // The direct kernels loop over 256-triangle batches.  While the batches fit
@@ -1409,7 +1419,10 @@ void voxelize(hipStream_t stream, const nlod_voxinfo* info, const float* d_tris,
         NLOD_LAUNCH_CHECK();
     }
     if (p.n_tri == 0) return;
-    auto workspace = [&](size_t bytes) { return no_alloc ? fixed : tile_workspace(stream, bytes); };
+    TileScratch* own = tiled && !no_alloc ? &tile_scratch(stream) : nullptr;
+    std::unique_lock<std::mutex> job;
+    if (own) job = std::unique_lock<std::mutex>(own->mu);
+    auto workspace = [&](size_t bytes) { return own ? own->ensure(stream, bytes) : fixed; };
     if (flags & NLOD_VOX_SOLID) launch_voxelize<true>(stream, p, geo, tiled, d_tris, d_table, workspace);
     else launch_voxelize<false>(stream, p, geo, tiled, d_tris, d_table, workspace);
 }
