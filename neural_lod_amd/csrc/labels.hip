@@ -258,10 +258,11 @@ __device__ __forceinline__ float uniform_at(uint64_t s, uint32_t n) {
 // registers, kCached triangles each, for all paths of the sample; longer lists
 // run on 64 lanes and read their rest at every ray.  A block draws its samples' voxels,
 // sorts them by G and its waves take them from an LDS counter, 64 / G samples at
-// a time and the longest lists first.  What bounds it: VALU issue and, for few
-// samples, the chain of the slowest sample.  16384 samples of 64 paths of that
-// pyramid: 93.9 ms with one lane per sample (its wave waits for the longest
-// list, and 256 waves leave the chip idle), 1.50 ms like this.
+// a time and the longest lists first.  What bounds it: the chains of the slowest
+// samples.  16384 samples of 64 paths of that pyramid: 93.9 ms with one lane per
+// sample (its wave waits for the longest list, and 256 waves leave the chip idle),
+// 1.50 ms like this; 2.9 of the 16 waves that a CU starts with are running on
+// average, and the VALU issues in 27% of the cycles.
 constexpr int kCached = 2;
 constexpr int kMaxBlockSamples = 64;
 

@@ -1396,9 +1396,14 @@ void voxelize(hipStream_t stream, const nlod_voxinfo* info, const float* d_tris,
     p.morton = (flags & NLOD_VOX_MORTON) ? 1 : 0;
     p.n_tri = info->n_triangles;
     TileGeo geo{};
-    // default: tiled for the solid fill (its row ranges make global atomics
-    // the bound of the direct kernel); the surface test is compute-bound
-    // either way and the direct kernel has no binning passes
+    // default: tiled for the solid fill, whose row ranges cost the direct kernel an
+    // atomic per word.  The surface test has fewer bits to set (29 M atomics for 1.5M
+    // triangles at 512^3, 145 M for 20M at 256^3, 1.5 M for 200k at 256^3, at 21 G/s at
+    // most: all of the first one's time, most of the second's, two thirds of the
+    // third's) and tests every voxel either way; setting them in LDS does not make up
+    // for the binning passes and the triangles' set-up in every tile that they meet:
+    // direct and tiled, 1000 triangles at 64^3 14 and 27 us, 200k at 256^3 106 and 135
+    // us, 1.5M at 512^3 1.36 and 2.50 ms, 20M at 256^3 7.9 and 8.5 ms
     const bool want = (flags & NLOD_VOX_TILED) || ((flags & NLOD_VOX_SOLID) && !(flags & NLOD_VOX_DIRECT));
     const bool tiled = p.n_tri > 0 && !p.morton && want &&
                        tile_geometry(p.G, p.n_tri, (flags & NLOD_VOX_TILED) != 0, (flags & NLOD_VOX_ACCUMULATE) != 0,

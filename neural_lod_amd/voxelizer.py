@@ -76,7 +76,7 @@ def voxelize(triangles: torch.Tensor, res: int, solid: bool = False, pad: bool =
     With ``info`` given, that box is used as is (no bounding-box pass).
     ``path`` picks the kernels ("direct": one triangle per lane with global
     atomics; "tiled": LDS tiles of voxel rows; "auto": tiled for larger
-    row-major jobs); all give identical bits."""
+    row-major solid jobs); all give identical bits."""
     t = _check_tris(triangles)
     words = table_words(res)
     if out is None:
