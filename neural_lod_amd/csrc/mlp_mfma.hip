@@ -387,14 +387,15 @@ __global__ __launch_bounds__(NT) void mlp_fwd_kernel(MlpArgs16 a, const half_t* 
     }
 }
 
-// ReLU networks with inputs up to 128 features (32 at width 128, where more
-// prefetched fragments would spill) take the prefetching kernels
+// ReLU networks with inputs up to 128 features (32 at width 128 with pairs of
+// tiles or blocks of 8 waves and more, where more prefetched fragments would
+// spill) take the prefetching kernels
 template <int W, int TT, int NT, typename Launch>
 void launch_fwd(const MlpArgs16& a, Launch&& launch) {
     if (a.act != ACT_RELU) return launch(mlp_fwd_kernel<W, TT, -1, 0, NT>, TT, NT);
     const uint32_t kc = a.k_padded / 32;
     if (kc == 1) return launch(mlp_fwd_kernel<W, TT, ACT_RELU, 1, NT>, TT, NT);
-    if constexpr (W < 128) {
+    if constexpr (W < 128 || NT == kBlock) {
         switch (kc) {
             case 2: return launch(mlp_fwd_kernel<W, TT, ACT_RELU, 2, NT>, TT, NT);
             case 3: return launch(mlp_fwd_kernel<W, TT, ACT_RELU, 3, NT>, TT, NT);
@@ -582,7 +583,15 @@ void mfma_mlp_forward(hipStream_t stream, const Layout& L, const void* packed, c
             // encoding: 141 -> 100 us, 106 us with 12), else 12 (158 -> 93 us, 99 us
             // with 8).  While one tile a wave covers the batch, one round of single
             // tiles is shorter (30000 queries: 42 -> 29.5 us, 33 us with pairs).
-            if (n_tiles <= 8 * (uint32_t)cu_count()) launch_fwd<128, 1, 512>(a, launch);
+            // Shallow networks, whose weights leave room for four blocks, or three
+            // that prefetch more than 32 inputs, keep blocks of 4 waves with single
+            // tiles (MLP alone, 2^19 queries, us with them and without: 1 hidden layer,
+            // 16 inputs 11.8 and 14.7, 40 inputs 16.2 and 20.5, 100 inputs 26.4 and
+            // 29.4; 2 hidden layers, 40 inputs 29.8 and 32.1, but 16 inputs 27.6 and
+            // 25.1 and 100 inputs, two blocks, 41.3 and 41.0).
+            if (smem <= 40 * 1024 || (smem <= 53 * 1024 && a.act == ACT_RELU && a.k_padded > 32 && a.k_padded <= 128))
+                launch_fwd<128, 1, kBlock>(a, launch);
+            else if (n_tiles <= 8 * (uint32_t)cu_count()) launch_fwd<128, 1, 512>(a, launch);
             else if (a.k_padded == 32) launch_fwd<128, 2, 512>(a, launch);
             else launch_fwd<128, 2, 768>(a, launch);
             break;

@@ -1,8 +1,8 @@
-"""FP16 network passes at the limits of their blocks: 128-wide networks without a
-hidden activation at the sizes where the block's shape changes (single tiles while
-8 waves a CU cover the batch, 32768 queries on 256 CUs; then pairs of tiles, on 8
-waves for 32 inputs and 12 for more), and a backward pass whose weights fill the
-LDS to the last byte.
+"""FP16 network passes at the limits of their blocks: 128-wide networks at the sizes
+where the block's shape changes (single tiles while 8 waves a CU cover the batch,
+32768 queries on 256 CUs; then pairs of tiles, on 8 waves for 32 inputs and 12 for
+more; single tiles on 4 waves for shallow networks, with 1 to 4 chunks of inputs
+loaded ahead), and a backward pass whose weights fill the LDS to the last byte.
 
 Against the MLP with FP16 weights and features, rounded to FP16 where the kernels
 round and summed in float64: a layer's FP32 sums may round to the next FP16 value
@@ -53,14 +53,15 @@ def _inputs(net, n, n_in, width, seed):
     return p, x
 
 
-@pytest.mark.parametrize("n_in,n_hidden", [(30, 4), (150, 3)])
-@pytest.mark.parametrize("n", [100, 32768, 32769, 40007])
-def test_wide_forward_without_activation(cuda, n_in, n_hidden, n):
-    print(f"case mlp fp16 in={n_in} hidden={n_hidden} n={n}", flush=True)
-    net = _net(128, n_hidden, n_in, 5, "None")
+@pytest.mark.parametrize("n_in,n_hidden,activation", [(30, 4, "None"), (150, 3, "None"), (30, 1, "None"), (30, 1, "ReLU"),
+                                                      (50, 2, "ReLU"), (90, 1, "ReLU"), (120, 1, "ReLU")])
+@pytest.mark.parametrize("n", [1, 100, 32768, 32769, 40007])
+def test_wide_forward(cuda, n_in, n_hidden, activation, n):
+    print(f"case mlp fp16 in={n_in} hidden={n_hidden} {activation} n={n}", flush=True)
+    net = _net(128, n_hidden, n_in, 5, activation)
     p, x = _inputs(net, n, n_in, 128, n)
     net.set_params(p)
-    ref = _forward(net, _matrices(net, p, 128, n_hidden), x, False)[1][:, :5]
+    ref = _forward(net, _matrices(net, p, 128, n_hidden), x, activation == "ReLU")[1][:, :5]
     err, scale = (net.inference(x).double() - ref).abs().max().item(), ref.abs().max().item()
     assert err <= 2e-3 * scale, f"error {err:.3e}, largest value {scale:.3e}"
 
